@@ -2,6 +2,7 @@
 
 from __future__ import annotations
 
+import functools
 import math
 from typing import Iterable
 
@@ -12,6 +13,8 @@ _ALLOWED = (np.float32, np.float64)
 
 def precision_from(precision) -> type:
     """Normalise a dtype-like to ``np.float32`` or ``np.float64``."""
+    if precision is np.float64 or precision is np.float32:
+        return precision
     dt = np.dtype(precision)
     if dt == np.float32:
         return np.float32
@@ -28,7 +31,10 @@ def c_literal(value: float, precision) -> str:
     constant with ``precision(value)``).
     """
     prec = precision_from(precision)
-    v = float(prec(value))
+    return _hex_literal(float(prec(value)), prec)
+
+
+def _hex_literal(v: float, prec) -> str:
     if math.isnan(v):
         return "__builtin_nan(\"\")" if prec is np.float64 else "__builtin_nanf(\"\")"
     if math.isinf(v):
@@ -51,10 +57,17 @@ def c_double(value: float) -> str:
 
 
 def c_array(values: Iterable[float], precision) -> str:
-    vals = list(values)
+    prec = precision_from(precision)
+    return _array_text(np.array(list(values), dtype=np.float64).tobytes(), prec)
+
+
+@functools.lru_cache(maxsize=2048)
+def _array_text(doubles: bytes, prec) -> str:
+    """The initialiser of these doubles (by their bits: -0.0 is not 0.0)."""
+    vals = np.frombuffer(doubles).astype(prec).tolist()
     if not vals:
         vals = [0.0]
-    return "{" + ", ".join(c_literal(v, precision) for v in vals) + "}"
+    return "{" + ", ".join(_hex_literal(v, prec) for v in vals) + "}"
 
 
 def c_int_array(values: Iterable[int]) -> str:

@@ -376,7 +376,7 @@ class BatchSolverKernel:
         mode = kernel_mode or self.kernel_mode
         name = {"plain": "cubie_integrate", "persistent": "cubie_integrate_persistent",
                 "record": "cubie_integrate_record", "adjoint": "cubie_adjoint"}[mode]
-        return kcache.get_module(spec.source(), spec.compile_options(), name)
+        return kcache.get_module_of_parts(spec.source_parts(), spec.compile_options(), name)
 
     def compile_only(self, duration: float = 1.0, per_run_rtol: bool = False) -> bytes:
         """Compile (or fetch from the cache) without touching a GPU."""
@@ -627,7 +627,8 @@ class BatchSolverKernel:
         if duration_per_run is not None:
             cols.append(torch.from_numpy(np.asarray(duration_per_run, dtype=np.float64)).to(dev))
         order = morton_order(cols)
-        o_host = order.cpu().numpy()
+        o_host = (order.cpu().numpy() if rtol_per_run is not None or duration_per_run is not None
+                  else None)
         d_i = d_i.index_select(1, order).contiguous()
         d_p = d_p.index_select(1, order).contiguous() if d_p.numel() else d_p
         rt = None if rtol_per_run is None else np.asarray(rtol_per_run)[o_host]
@@ -713,10 +714,14 @@ class BatchSolverKernel:
         shapes = self.output_shapes(timing, dur_for_rows, n_runs)
         staged = self.run_major_rows(adjoint)
         outs = {}
+        # one cleared block: the persistent kernel's queue counter and the
+        # one-element stand-ins of inactive outputs
+        cleared = torch.zeros(4, dtype=torch.int32, device=dev)
+        counter = cleared[:1]
         for k, shp in shapes.items():
             dt_ = torch.int32 if k == "iteration_counters" else tdt
             if shp[0] * shp[1] == 0:
-                outs[k] = torch.zeros(1, dtype=dt_, device=dev)
+                outs[k] = cleared[2:].view(dt_)[:1]
             elif staged and k in ROW_OUTPUTS:
                 # (run, time, variable) staging; transposed after the launch
                 outs[k] = torch.zeros((shp[2], shp[0], shp[1]), dtype=dt_, device=dev)
@@ -731,7 +736,6 @@ class BatchSolverKernel:
         rtol_d = to_dev(np.asarray(rtol_per_run), tdt) if per_run_rtol else None
         dur_d = (torch.from_numpy(np.asarray(duration_per_run, dtype=np.float64)).to(dev)
                  if duration_per_run is not None else None)
-        counter = torch.zeros(1, dtype=torch.int32, device=dev)
         # [2][n_runs] Newton / Krylov iterations of every solve (optional)
         tally = torch.zeros((4, n_runs), dtype=torch.int32, device=dev) if work_tally else None
         table_d = (torch.tensor(timing.save_times, dtype=torch.float64, device=dev)

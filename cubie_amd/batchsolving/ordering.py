@@ -30,15 +30,17 @@ def morton_order(columns: List["object"]):
     the Morton key of the given (n_runs,) float tensors."""
     import torch
     cols = []
-    for c in columns:
-        c = c.to(torch.float64)
-        lo, hi = c.min(), c.max()
-        span = float(hi - lo)
-        scale = max(float(c.abs().max()), 1e-300)
-        if span > 1e-12 * scale:
-            cols.append(((c - lo) / span, span / scale))
     n = int(columns[0].numel()) if columns else 0
     dev = columns[0].device if columns else None
+    if columns:
+        wide = [c.to(torch.float64) for c in columns]
+        # every column's range in one transfer to the host
+        ranges = torch.stack([torch.stack((c.min(), c.max(), c.abs().max())) for c in wide])
+        for c, (lo, hi, top) in zip(wide, ranges.tolist()):
+            span = hi - lo
+            scale = max(top, 1e-300)
+            if span > 1e-12 * scale:
+                cols.append(((c - lo) / span, span / scale))
     if not cols:
         return torch.arange(n, device=dev)
     cols.sort(key=lambda cs: -cs[1])

@@ -239,19 +239,19 @@ class Solver:
             dout, ms, info = self.kernel.run(inits, params, duration=duration,
                                              warmup=settling_time, t0=t0, blocksize=blocksize,
                                              rtol_per_run=rtol_per_run,
-                                             duration_per_run=duration_per_run, timed=True)
+                                             duration_per_run=duration_per_run,
+                                             timed=not on_device)
             self._last = info
             if on_device:
                 import torch
                 return DeviceSolveResult(dout, torch.cuda.current_stream(), oc.save_time, active)
-            host = {k: getattr(dout, k).cpu().numpy() for k in
-                    ("state", "observables", "state_summaries", "observable_summaries",
-                     "iteration_counters", "status_codes")}
-            sh = info["shapes"]
-            for k in ("state", "observables", "state_summaries", "observable_summaries",
-                      "iteration_counters"):
-                host[k] = (host[k].reshape(sh[k]) if np.prod(sh[k]) > 0
-                           else np.zeros(sh[k], dtype=host[k].dtype))
+            host = {"status_codes": dout.status_codes.cpu().numpy()}
+            for k, sh in info["shapes"].items():
+                if np.prod(sh) > 0:
+                    host[k] = getattr(dout, k).cpu().numpy().reshape(sh)
+                else:
+                    host[k] = np.zeros(sh, dtype=np.int32 if k == "iteration_counters"
+                                       else self.system.precision)
         return SolveResult(host["state"], host["observables"], host["state_summaries"],
                            host["observable_summaries"], host["status_codes"],
                            host["iteration_counters"], save_time=oc.save_time, active=active,

@@ -11,6 +11,7 @@ and controller constant into the gfx950 code.
 
 from __future__ import annotations
 
+import functools
 import hashlib
 import os
 from dataclasses import dataclass, field
@@ -35,6 +36,14 @@ DEVICE_HEADERS = [
     "detmath.hpp", "common.hpp", "drivers.hpp", "controllers.hpp", "outputs.hpp", "linear.hpp",
     "erk.hpp", "dirk.hpp", "firk.hpp", "rosenbrock.hpp", "euler_implicit.hpp", "loop.hpp",
 ]
+
+
+@functools.lru_cache(maxsize=None)
+def _header_text(path: str) -> str:
+    """A header of the package (read once per process)."""
+    with open(path) as f:
+        return f.read()
+
 
 # Families whose mixed-precision mode solves the Krylov systems in FP32.
 FP32_KRYLOV_FAMILIES = ("dirk", "backwards_euler", "backwards_euler_pc", "crank_nicolson")
@@ -506,24 +515,30 @@ class KernelSpec:
         )
 
     def source(self) -> str:
+        return "\n".join(self.source_parts())
+
+    def source_parts(self) -> Tuple[str, ...]:
+        """The translation unit in pieces. The settings (``config_struct``)
+        are written afresh on every call, so a changed setting is always
+        seen; the generated system and the headers, which are most of the
+        text and take far longer to make, come from their own caches
+        (``SystemCodegen.emit_cached``)."""
         parts = ["// Generated translation unit: configuration + system + device library.",
                  "#define CUBIE_DEVICE_COMPILE 1"]
         if self.resolved_placement == "memory":
             parts.append('#define CUBIE_UNROLL _Pragma("unroll 1")')
-        with open(os.path.join(INCLUDE, "cubie_hip.h")) as f:
-            parts.append(f.read())
+        parts.append(_header_text(os.path.join(INCLUDE, "cubie_hip.h")))
         parts.append(self.config_struct())
         parts.append("using real = Cfg::real;")
         if self.adjoint:
             self.check_adjoint()
         gen = SystemCodegen(self.system, self.precision, adjoint=self.adjoint)
-        parts.append(gen.emit())
+        parts.append(gen.emit_cached())
         self.op_counts = gen.op_counts
         parts.append(self.plugin_hooks())
         for h in DEVICE_HEADERS:
-            with open(os.path.join(CSRC, "device", h)) as f:
-                parts.append(f"// ---- {h} ----")
-                parts.append(f.read())
+            parts.append(f"// ---- {h} ----")
+            parts.append(_header_text(os.path.join(CSRC, "device", h)))
         stepper = FAMILY_STEPPER[self.algorithm.family]
         bs = int(self.block_size)
         attrs = f"__launch_bounds__({bs})"
@@ -537,9 +552,8 @@ class KernelSpec:
             f"extern \"C\" __global__ void {attrs} cubie_integrate_persistent(cubie_solve_args a) {{\n"
             "  cubie::integrate_persistent<Cfg, System, StepperT>(a);\n}\n")
         if self.adjoint:
-            with open(os.path.join(CSRC, "device", "adjoint.hpp")) as f:
-                parts.append("// ---- adjoint.hpp ----")
-                parts.append(f.read())
+            parts.append("// ---- adjoint.hpp ----")
+            parts.append(_header_text(os.path.join(CSRC, "device", "adjoint.hpp")))
             adj = FAMILY_ADJOINT[self.algorithm.family]
             parts.append(
                 f"using AdjointT = cubie::{adj}<Cfg, System>;\n"
@@ -547,7 +561,7 @@ class KernelSpec:
                 "  cubie::integrate_record<Cfg, System, StepperT>(a);\n}\n"
                 f"extern \"C\" __global__ void {attrs} cubie_adjoint(cubie_adjoint_args a) {{\n"
                 "  cubie::adjoint_backward<Cfg, System, AdjointT>(a);\n}\n")
-        return "\n".join(parts)
+        return tuple(parts)
 
     def check_adjoint(self) -> None:
         """The discrete adjoint covers the explicit RK and Rosenbrock-W

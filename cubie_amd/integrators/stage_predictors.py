@@ -20,6 +20,7 @@ within the tableau's calibrated ceiling for the precision.
 
 from __future__ import annotations
 
+import functools
 from typing import Tuple
 
 import numpy as np
@@ -62,8 +63,13 @@ def readahead_matrix(nodes, ratio: float, samples) -> np.ndarray:
 
 
 def supports_prediction(tableau) -> bool:
-    nodes = np.asarray(tableau.c, dtype=np.float64)
-    samples = sample_stages(tableau.c)
+    return _supports_prediction(tuple(float(x) for x in tableau.c))
+
+
+@functools.lru_cache(maxsize=64)
+def _supports_prediction(c: Tuple[float, ...]) -> bool:
+    nodes = np.asarray(c, dtype=np.float64)
+    samples = sample_stages(c)
     k = len(samples)
     amp = float(np.abs(readahead_matrix(nodes, 1.0, samples)).sum(axis=1).max())
     g = 0.5 * (leggauss(k)[0] + 1.0)
@@ -73,9 +79,14 @@ def supports_prediction(tableau) -> bool:
 
 def ratio_coefficients(tableau) -> np.ndarray:
     """(powers, stages, stages) with P(r) = sum_p C[p] r^(p+1)."""
-    nodes = np.asarray(tableau.c, dtype=np.float64)
+    return _ratio_coefficients(tuple(float(x) for x in tableau.c)).copy()
+
+
+@functools.lru_cache(maxsize=64)
+def _ratio_coefficients(c: Tuple[float, ...]) -> np.ndarray:
+    nodes = np.asarray(c, dtype=np.float64)
     s = nodes.size
-    samples = sample_stages(tableau.c)
+    samples = sample_stages(c)
     dn = [nodes[i] for i in samples]
     k = len(dn)
     shift = P.Polynomial([1.0, 1.0])
@@ -85,9 +96,9 @@ def ratio_coefficients(tableau) -> np.ndarray:
         coef = P.polyfromroots(others)
         coef = coef / P.polyval(dn[bi], coef)
         shifted = P.Polynomial(coef)(shift)
-        c = np.zeros(k)
-        c[: shifted.coef.size] = shifted.coef
-        weights.append(c)
+        row = np.zeros(k)
+        row[: shifted.coef.size] = shifted.coef
+        weights.append(row)
     out = np.zeros((k, s, s))
     for p in range(k):
         for ti in range(s):

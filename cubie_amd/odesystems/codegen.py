@@ -42,6 +42,7 @@ from __future__ import annotations
 
 import math
 import re
+import threading
 from typing import Dict, Iterable, List, Sequence, Tuple
 
 import numpy as np
@@ -394,6 +395,11 @@ def jacobian_nonzeros(system) -> List[Tuple[int, int]]:
     return out
 
 
+# generated texts kept per system (precisions x with / without the adjoint)
+EMITTED_VARIANTS = 8
+_emitted_lock = threading.Lock()
+
+
 class SystemCodegen:
     """Generate the ``System`` struct of device functions for one system."""
 
@@ -401,8 +407,37 @@ class SystemCodegen:
         self.system = system
         self.precision = precision or system.precision
         self.adjoint = bool(adjoint)
-        self.printer = HipPrinter(self.precision, system.user_functions)
+        self._printer = None
         self.op_counts: Dict[str, Dict[str, int]] = {}
+
+    @property
+    def printer(self) -> "HipPrinter":
+        if self._printer is None:
+            self._printer = HipPrinter(self.precision, self.system.user_functions)
+        return self._printer
+
+    def emit_cached(self) -> str:
+        """``emit()``, kept on the system for an unchanged system: the key
+        holds the values the text is generated from (equations, constants,
+        user functions, names, precision), so a changed constant generates
+        anew. The last few variants are kept."""
+        s = self.system
+        key = (self.precision, self.adjoint, s.name,
+               tuple((a.lhs, a.rhs, a.kind) for a in s.assignments),
+               tuple(s.constants.items()), tuple(sorted(s.user_functions.items())),
+               tuple(s.state_names), tuple(s.parameter_names), tuple(s.driver_names),
+               tuple(s.observable_names))
+        cache = s.__dict__.setdefault("_emitted", {})
+        hit = cache.get(key)
+        if hit is None:
+            hit = (self.emit(), self.op_counts)
+            with _emitted_lock:
+                while len(cache) >= EMITTED_VARIANTS:
+                    del cache[next(iter(cache))]
+                cache[key] = hit
+        text, counts = hit
+        self.op_counts = {k: dict(v) for k, v in counts.items()}
+        return text
 
     # -- helpers -------------------------------------------------------------
     def _bindings(self, use_drivers=True) -> List[str]:

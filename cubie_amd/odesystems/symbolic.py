@@ -344,6 +344,7 @@ class SymbolicODE:
         other._state_defaults = dict(self._state_defaults)
         other._parameter_defaults = dict(self._parameter_defaults)
         other._constants = dict(self._constants)
+        other.__dict__.pop("_emitted", None)
         return other
 
     def set_constants(self, updates: Mapping[str, float]) -> None:

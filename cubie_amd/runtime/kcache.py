@@ -14,6 +14,7 @@ from __future__ import annotations
 import hashlib
 import os
 import tempfile
+import threading
 from typing import Dict, List, Tuple
 
 from . import native
@@ -23,6 +24,12 @@ DEFAULT_DIR = os.path.join(_PKG, "_kernel_cache")
 
 _memory: Dict[str, bytes] = {}
 _modules: Dict[Tuple[str, str], "native.Module"] = {}
+# (pieces of a translation unit, options, kernel) -> module: the pieces are
+# compared by value, most of them being the very same string objects, which
+# spares joining and hashing the whole text on each launch
+_by_parts: Dict[tuple, "native.Module"] = {}
+PARTS_KEPT = 256
+_parts_lock = threading.Lock()
 
 
 def cache_dir() -> str:
@@ -66,3 +73,17 @@ def get_module(source: str, options: List[str], kernel: str) -> "native.Module":
     if mk not in _modules:
         _modules[mk] = native.Module(code, kernel)
     return _modules[mk]
+
+
+def get_module_of_parts(parts: Tuple[str, ...], options: List[str],
+                        kernel: str) -> "native.Module":
+    """``get_module`` of the translation unit the pieces make."""
+    pk = (parts, tuple(options), kernel)
+    mod = _by_parts.get(pk)
+    if mod is None:
+        mod = get_module("\n".join(parts), options, kernel)
+        with _parts_lock:
+            while len(_by_parts) >= PARTS_KEPT:
+                del _by_parts[next(iter(_by_parts))]
+            _by_parts[pk] = mod
+    return mod

@@ -1,0 +1,44 @@
+"""The kept pieces of a translation unit follow every setting they depend on."""
+
+import numpy as np
+
+import cubie_amd as ca
+from cubie_amd._utils import c_array, c_literal
+from systems import hodgkin_huxley, lorenz
+
+
+def _source(solver):
+    return solver.kernel.spec_for(1.0).source()
+
+
+def test_changed_constant_and_controller_are_seen():
+    sysm = hodgkin_huxley(np.float64)
+    solver = ca.Solver(sysm, algorithm="l_stable_dirk_3", dt=0.01, save_every=0.5,
+                       output_types=["state"])
+    first = _source(solver)
+    assert _source(solver) == first
+    sysm.set_constants({"ENa": 55.0})
+    second = _source(solver)
+    assert second != first
+    assert second == _source(ca.Solver(sysm, algorithm="l_stable_dirk_3", dt=0.01,
+                                       save_every=0.5, output_types=["state"]))
+    sysm.set_constants({"ENa": 50.0})
+    assert _source(solver) == first
+    solver.kernel.controller.dt = 0.02
+    assert _source(solver) != first
+
+
+def test_precisions_do_not_share_text():
+    a = lorenz(np.float64)
+    s64 = _source(ca.Solver(a, algorithm="tsit5", save_every=0.5, output_types=["state"]))
+    s32 = _source(ca.Solver(a.with_precision(np.float32), algorithm="tsit5", save_every=0.5,
+                            output_types=["state"]))
+    assert s64 != s32
+    assert s64 == _source(ca.Solver(lorenz(np.float64), algorithm="tsit5", save_every=0.5,
+                                    output_types=["state"]))
+
+
+def test_array_text_keeps_the_sign_of_zero():
+    for prec in (np.float32, np.float64):
+        vals = [0.0, -0.0, 1.0 / 3.0, float("inf"), -1e-320]
+        assert c_array(vals, prec) == "{" + ", ".join(c_literal(v, prec) for v in vals) + "}"
