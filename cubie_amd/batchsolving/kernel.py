@@ -64,6 +64,9 @@ def _torch():
 # operation; at relative tolerances below this floor it is of the order of the
 # error estimate itself, so the compensated mode hands such runs to FP64
 COMPENSATED_RTOL_FLOOR = 1e-6
+# LDS of the row ring: bytes per lane, and per workgroup at most
+ROW_RING_LANE = 160
+ROW_RING_LDS = 80 * 1024
 OUTPUT_FIELDS = ("state", "observables", "state_summaries", "observable_summaries",
                  "iteration_counters", "status_codes", "work_tally")
 
@@ -324,23 +327,68 @@ class BatchSolverKernel:
                                  f"({duration}), so this loop will produce no summary outputs")
 
     # -- spec / module --------------------------------------------------------
-    def run_major_rows(self, adjoint: bool = False) -> bool:
-        """Whether per-row outputs are staged run-major (see outputs.hpp
-        row_index): adaptive algorithms with time-domain outputs, unless
-        output_staging="direct"; never for the adjoint's recording pass."""
+    def _rows_out_of_step(self, adjoint: bool) -> bool:
+        """Whether the lanes of a wavefront reach a save time at different
+        loop iterations (adaptive runs with time-domain outputs), so that
+        rows are buffered or staged; never with output_staging="direct" nor
+        in the adjoint's recording pass."""
         return (self.output_staging == "auto" and not adjoint and self.algorithm.is_adaptive
                 and self.controller.is_adaptive and self.output_config.time_domain_outputs)
 
+    def row_ring(self, adjoint: bool = False, kernel_mode: Optional[str] = None,
+                 block_size: Optional[int] = None) -> int:
+        """Rows of LDS per lane for the plain kernel's RowRing (outputs.hpp),
+        or 0. The persistent kernel's lanes hold scattered runs, so it stages
+        run-major instead.
+
+        The largest power of two within 160 bytes a lane: four 256-lane
+        workgroups share a CU's 160 KB then, so the ring does not lower the
+        occupancy of a kernel that needs up to 128 VGPRs. Wider rows get two
+        slots as long as a workgroup's ring fits in half a CU's LDS; beyond
+        that rows are staged, as they are where the vectors live in the
+        private segment: a step there costs so much traffic that staging is
+        lost in it (20 states x 50,000 runs: 57 ms, of which the transpose
+        0.16 ms), while lanes that wait for one another are not (60 ms)."""
+        if (kernel_mode or self.kernel_mode) != "plain" or not self._rows_out_of_step(adjoint):
+            return 0
+        if KernelSpec.placement_of(self.buffer_placement, self.system.num_states) != "registers":
+            return 0
+        oc = self.output_config
+        item = np.dtype(self.precision).itemsize
+        width = oc.state_output_width if (oc.save_state or oc.save_time) else 0
+        width += oc.n_saved_observables if oc.save_observables else 0
+        row = item * width + (16 if oc.save_counters else 0)
+        lanes = int(block_size or self.block_size)
+        if row == 0 or 2 * row * lanes > ROW_RING_LDS:
+            return 0
+        slots = 2
+        while 2 * slots * row <= ROW_RING_LANE and 2 * slots * row * lanes <= ROW_RING_LDS:
+            slots *= 2
+        return slots
+
+    def run_major_rows(self, adjoint: bool = False, kernel_mode: Optional[str] = None,
+                       block_size: Optional[int] = None) -> bool:
+        """Whether per-row outputs are staged run-major (see outputs.hpp
+        row_index) and transposed after the launch: rows out of step that no
+        ring takes."""
+        return (self._rows_out_of_step(adjoint)
+                and not self.row_ring(adjoint, kernel_mode, block_size))
+
     def spec_for(self, duration: float, per_run_rtol: bool = False, adjoint: bool = False,
-                 adj_ckpt_every: int = 32, block_size: Optional[int] = None) -> KernelSpec:
+                 adj_ckpt_every: int = 32, block_size: Optional[int] = None,
+                 kernel_mode: Optional[str] = None) -> KernelSpec:
         """The kernel specification for one run; ``block_size`` (default: the
-        configured one) is compiled into the kernel's launch bounds."""
+        configured one) is compiled into the kernel's launch bounds, and the
+        way rows are written follows ``kernel_mode`` (default: the configured
+        one)."""
         timing = self.timing.with_duration(duration)
         block_size = int(block_size or self.block_size)
+        staged = self.run_major_rows(adjoint, kernel_mode, block_size)
+        ring = self.row_ring(adjoint, kernel_mode, block_size)
         key = (timing.summarise_every, timing.sample_summaries_every, per_run_rtol,
                self.precision_mode, self.fp_contract, block_size, self.deterministic_pow,
                self.waves_per_eu, bool(adjoint), int(adj_ckpt_every), self.compensated_rhs,
-               self.buffer_placement, self.run_major_rows(adjoint), self.compensated_stage_rhs,
+               self.buffer_placement, staged, ring, self.compensated_stage_rhs,
                self.sparse_jacobian, self.compensated_jacobian)
         if key not in self._spec_cache:
             self._spec_cache[key] = KernelSpec(
@@ -352,7 +400,7 @@ class BatchSolverKernel:
                 deterministic_pow=self.deterministic_pow, waves_per_eu=self.waves_per_eu,
                 adjoint=bool(adjoint), adj_ckpt_every=int(adj_ckpt_every),
                 compensated_rhs=self.compensated_rhs, buffer_placement=self.buffer_placement,
-                run_major_rows=self.run_major_rows(adjoint),
+                run_major_rows=staged, row_ring=ring,
                 compensated_stage_rhs=self.compensated_stage_rhs,
                 sparse_jacobian=self.sparse_jacobian,
                 compensated_jacobian=self.compensated_jacobian)
@@ -407,11 +455,12 @@ class BatchSolverKernel:
         """
         if _compile_only():
             dur = float(np.float64(duration))
-            spec = self.spec_for(dur, rtol_per_run is not None, block_size=blocksize)
+            spec = self.spec_for(dur, rtol_per_run is not None, block_size=blocksize,
+                                 kernel_mode=kernel_mode)
             kcache.get_code(spec.source(), spec.compile_options())
             if self._fp64_fallback_runs(inits, rtol_per_run) is not None:
                 twin = self.fp64_twin().spec_for(dur, rtol_per_run is not None,
-                                                 block_size=blocksize)
+                                                 block_size=blocksize, kernel_mode=kernel_mode)
                 kcache.get_code(twin.source(), twin.compile_options())
             raise CompileOnly(spec)
         if blocksize is not None and not (1 <= int(blocksize) <= 1024 and int(blocksize) % 64 == 0):
@@ -431,11 +480,12 @@ class BatchSolverKernel:
                 t_start.record()
             inits, params, rtol_per_run, duration_per_run, order = self._sorted_inputs(
                 inits, params, rtol_per_run, duration_per_run)
-        st = self.setup(inits, params, duration, warmup, t0, rtol_per_run, duration_per_run,
-                        work_tally=work_tally)
-        # a requested block size is compiled into the kernel's launch bounds
-        spec = self.spec_for(st["duration"], st["per_run_rtol"], block_size=blocksize)
         mode = kernel_mode or self.kernel_mode
+        st = self.setup(inits, params, duration, warmup, t0, rtol_per_run, duration_per_run,
+                        work_tally=work_tally, kernel_mode=mode, block_size=blocksize)
+        # a requested block size is compiled into the kernel's launch bounds
+        spec = self.spec_for(st["duration"], st["per_run_rtol"], block_size=blocksize,
+                             kernel_mode=mode)
         mod = self.module(spec, mode)
         n_runs, args = st["n_runs"], st["args"]
         block = spec.block_size
@@ -671,9 +721,11 @@ class BatchSolverKernel:
 
     def setup(self, inits, params, duration: float, warmup: float = 0.0, t0: float = 0.0,
               rtol_per_run=None, duration_per_run=None, rows_duration=None,
-              work_tally: bool = False, adjoint: bool = False) -> dict:
+              work_tally: bool = False, adjoint: bool = False,
+              kernel_mode: Optional[str] = None, block_size: Optional[int] = None) -> dict:
         """Validate the run, place inputs on the device, allocate the outputs
-        and fill the kernel's argument block (``native.SolveArgs``)."""
+        (the kernel writes every row and window) and fill the kernel's
+        argument block (``native.SolveArgs``)."""
         torch = _torch()
         prec = self.precision
         tdt = torch.float32 if prec is np.float32 else torch.float64
@@ -712,7 +764,7 @@ class BatchSolverKernel:
             raise ValueError("duration_per_run requires save_last / summary-free outputs")
 
         shapes = self.output_shapes(timing, dur_for_rows, n_runs)
-        staged = self.run_major_rows(adjoint)
+        staged = self.run_major_rows(adjoint, kernel_mode, block_size)
         outs = {}
         # one cleared block: the persistent kernel's queue counter and the
         # one-element stand-ins of inactive outputs
@@ -724,10 +776,10 @@ class BatchSolverKernel:
                 outs[k] = cleared[2:].view(dt_)[:1]
             elif staged and k in ROW_OUTPUTS:
                 # (run, time, variable) staging; transposed after the launch
-                outs[k] = torch.zeros((shp[2], shp[0], shp[1]), dtype=dt_, device=dev)
+                outs[k] = torch.empty((shp[2], shp[0], shp[1]), dtype=dt_, device=dev)
             else:
-                outs[k] = torch.zeros(shp, dtype=dt_, device=dev)
-        status = torch.zeros(n_runs, dtype=torch.int32, device=dev)
+                outs[k] = torch.empty(shp, dtype=dt_, device=dev)
+        status = torch.empty(n_runs, dtype=torch.int32, device=dev)
         coeffs = None
         if self.system.num_drivers > 0:
             if self.driver_interpolator is None:
@@ -849,8 +901,9 @@ class BatchSolverKernel:
 
         def make_slot(m):
             st = self.setup(inits[:, :m], params[:, :m] if params.size else params, duration,
-                            warmup, t0, sl(rtol, 0, m), sl(dpr, 0, m), rows_duration=rows_dur)
-            spec = self.spec_for(st["duration"], st["per_run_rtol"])
+                            warmup, t0, sl(rtol, 0, m), sl(dpr, 0, m), rows_duration=rows_dur,
+                            kernel_mode=mode)
+            spec = self.spec_for(st["duration"], st["per_run_rtol"], kernel_mode=mode)
             mod = self.module(spec, mode)
             block = spec.block_size
             if mode == "plain":

@@ -300,7 +300,7 @@ __device__ __forceinline__ void integrate_record(const cubie_adjoint_args& A) {
     while (!it.advance(a)) {
     }
     const long long N = a.n_runs;
-    a.status_out[run] = it.status | (it.tape.full ? ST_TAPE_FULL : 0);
+    it.finish(a, it.tape.full ? ST_TAPE_FULL : 0);
     A.tape_info[run] = int(it.tape.steps);
     A.tape_info[N + run] = int(it.save_idx);
     A.tape_info[2 * N + run] = int(it.update_idx);

@@ -9,6 +9,10 @@
 #ifndef __forceinline__
 #define __forceinline__ inline __attribute__((always_inline))
 #endif
+// the host build of the device library runs one lane at a time
+#ifndef __shared__
+#define __shared__ static thread_local
+#endif
 
 // Buffer placement of the per-system vectors. With register placement (the
 // default) every loop over a vector is unrolled, so each element has a

@@ -102,7 +102,9 @@ CUBIE_UNROLL
 };
 
 // Record = true: the adjoint's recording pass (fills a Tape as it goes).
-template <typename Cfg, typename Sys, typename Stepper, bool Record = false>
+// Rows: where saved rows go (DirectRows or RowRing, outputs.hpp).
+template <typename Cfg, typename Sys, typename Stepper, bool Record = false,
+          typename Rows = DirectRows<Cfg>>
 struct Integrator {
     using real = typename Cfg::real;
     using nreal = typename Cfg::norm_real;
@@ -113,6 +115,7 @@ struct Integrator {
     Stepper stepper;
     Controller<Cfg> ctrl;
     Summaries<Cfg> summ;
+    Rows rows;
     Vec<real, n> state, proposal;
     Vec<real, (Cfg::kahan_state ? n : 1)> state_c;   // Kahan compensation of state
     Vec<real, Cfg::n_error> error;
@@ -189,7 +192,7 @@ CUBIE_UNROLL
             if constexpr (Cfg::save_table) next_save = table_save(a, 1);
             else if constexpr (Cfg::save_regularly) next_save = real(next_save + Cfg::save_every);
             if constexpr (Cfg::summarise_regularly) next_update = real(Cfg::sample_summaries_every + next_update);
-            save_state<Cfg>(a, run, save_idx, state, ctx.observables, counters_since_save, t_prec);
+            rows.save(a, run, save_idx, state, ctx.observables, counters_since_save, t_prec);
             save_idx += 1;
             t_last_save = t_prec;
             if constexpr (summarise) summ.save(a, run, summary_idx);  // resets the window buffers
@@ -238,7 +241,7 @@ CUBIE_UNROLL
                 // to the working precision). The reference leaves that row
                 // unwritten (ode_loop.py:736-740); the state reached is the
                 // final state, so it is saved as the last row.
-                save_state<Cfg>(a, run, save_idx, state, ctx.observables, counters_since_save,
+                rows.save(a, run, save_idx, state, ctx.observables, counters_since_save,
                                 t_prec);
                 save_idx += 1;
                 t_last_save = t_prec;
@@ -353,7 +356,7 @@ CUBIE_UNROLL
         if (do_save) {
             if constexpr (Cfg::save_table) next_save = table_save(a, save_idx + 1);
             else if constexpr (Cfg::save_regularly) next_save += Cfg::save_every;
-            save_state<Cfg>(a, run, save_idx, state, ctx.observables, counters_since_save, t_prec);
+            rows.save(a, run, save_idx, state, ctx.observables, counters_since_save, t_prec);
             save_idx += 1;
             t_last_save = t_prec;
             if constexpr (Cfg::save_counters) {
@@ -375,6 +378,19 @@ CUBIE_UNROLL
         return false;
     }
 
+    // The run is over: its status and tally, and zeros for the rows and
+    // windows it did not reach (window 0 was written at the start of a run
+    // without settling time).
+    __device__ __forceinline__ void finish(const cubie_solve_args& a, int extra_status = 0) const {
+        a.status_out[run] = status | extra_status;
+        write_tally(a);
+        rows.zero_tail(a, run, save_idx);
+        if constexpr (summarise) {
+            const long long written = real(a.warmup) == real(0) ? 1 : 0;
+            summ.zero_tail(a, run, summary_idx > written ? summary_idx : written);
+        }
+    }
+
     // Newton iterations and Krylov iterations of every solve of every
     // attempted step, attempted steps and rejected steps, [4][n_runs] (an
     // engine extension: the work the algorithmic flop count of a run is
@@ -393,12 +409,29 @@ template <typename Cfg, typename Sys, typename Stepper>
 __device__ __forceinline__ void integrate_plain(const cubie_solve_args& a) {
     const long long run = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (run >= a.n_runs) return;
-    Integrator<Cfg, Sys, Stepper> it;
-    it.begin(a, run);
-    while (!it.advance(a)) {
+    if constexpr (Cfg::row_ring > 0) {
+        using Ring = RowRing<Cfg>;
+        constexpr int waves = Cfg::block_size / Ring::lanes;
+        constexpr int n_vals = waves * Ring::vals_per_wave;
+        constexpr int n_counts = waves * Ring::counts_per_wave;
+        __shared__ typename Cfg::io_real ring_vals[n_vals > 0 ? n_vals : 1];
+        __shared__ int ring_counts[n_counts > 0 ? n_counts : 1];
+        Integrator<Cfg, Sys, Stepper, false, Ring> it;
+        it.rows.bind(a, run, ring_vals, ring_counts);
+        it.begin(a, run);
+        bool done = false;
+        do {
+            if (!done && it.save_idx < it.rows.limit) done = it.advance(a);
+            it.rows.flush(a, it.save_idx, done);
+        } while (!wave_all(done));
+        it.finish(a);
+    } else {
+        Integrator<Cfg, Sys, Stepper> it;
+        it.begin(a, run);
+        while (!it.advance(a)) {
+        }
+        it.finish(a);
     }
-    a.status_out[run] = it.status;
-    it.write_tally(a);
 }
 
 // Wave-aggregated ticket: every lane with want=true receives a distinct run
@@ -424,10 +457,7 @@ __device__ __forceinline__ void integrate_persistent(const cubie_solve_args& a) 
     while (__any(active ? 1 : 0)) {
         bool done = false;
         if (active) done = it.advance(a);
-        if (active && done) {
-            a.status_out[it.run] = it.status;
-            it.write_tally(a);
-        }
+        if (active && done) it.finish(a);
         // Lanes that just finished take the next system of the batch.
         const long long next = grab_runs(a.work_counter, active && done);
         if (active && done) {

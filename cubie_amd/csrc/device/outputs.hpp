@@ -9,8 +9,10 @@
 //
 // Every store goes to [row][column][run] with the run index fastest, so a
 // wave that saves on the same loop iteration writes whole cache lines.
+// Adaptive runs do not: they go through RowRing, or are staged run-major.
 // Stores beyond the allocated rows are dropped (the host sizes the rows so
-// this never triggers in a well-formed run).
+// this never triggers in a well-formed run); rows and windows a run ended
+// before are written as zeros, so the host hands over uninitialised arrays.
 #pragma once
 
 namespace cubie {
@@ -262,6 +264,24 @@ CUBIE_UNROLL
         }
     }
 
+    // Windows [first, summary_rows) of a run that ended early read zero.
+    __device__ __forceinline__ static void zero_tail(const cubie_solve_args& a, long long run,
+                                                     long long first) {
+        constexpr int OH = Cfg::summ_out_height;
+        const long long N = a.n_runs;
+        using io_real = typename Cfg::io_real;
+        for (long long row = first; row < a.summary_rows; ++row) {
+            if constexpr (Cfg::summarise_state) {
+                io_real* out = static_cast<io_real*>(a.state_summ_out);
+                for (int k = 0; k < NS * OH; ++k) out[(row * (NS * OH) + k) * N + run] = io_real(0);
+            }
+            if constexpr (Cfg::summarise_obs) {
+                io_real* out = static_cast<io_real*>(a.obs_summ_out);
+                for (int k = 0; k < NO * OH; ++k) out[(row * (NO * OH) + k) * N + run] = io_real(0);
+            }
+        }
+    }
+
     // Flush every window buffer to its output row (or only reset, when
     // `row` is past the allocation, as the reference's initial call does).
     __device__ __forceinline__ void save(const cubie_solve_args& a, long long run, long long row) {
@@ -342,5 +362,152 @@ CUBIE_UNROLL
         for (int k = 0; k < 4; ++k) a.counters_out[row_index<Cfg>(a, run, row, 4, k)] = counters[k];
     }
 }
+
+// Row sink of the integrator: each saved row straight to its place.
+template <typename Cfg>
+struct DirectRows {
+    template <typename S, typename O>
+    __device__ __forceinline__ void save(const cubie_solve_args& a, long long run, long long row,
+                                         const S& state, const O& obs, const int* counters,
+                                         typename Cfg::real t_prec) {
+        save_state<Cfg>(a, run, row, state, obs, counters, t_prec);
+    }
+    // Rows [first, out_rows) of a run that ended early read zero.
+    __device__ __forceinline__ void zero_tail(const cubie_solve_args& a, long long run,
+                                              long long first) const {
+        using io_real = typename Cfg::io_real;
+        constexpr int W = Cfg::n_saved_states + (Cfg::save_time ? 1 : 0);
+        for (long long row = first; row < a.out_rows; ++row) {
+            if constexpr (Cfg::save_state || Cfg::save_time) {
+                io_real* out = static_cast<io_real*>(a.state_out);
+                for (int k = 0; k < W; ++k) out[row_index<Cfg>(a, run, row, W, k)] = io_real(0);
+            }
+            if constexpr (Cfg::save_obs) {
+                io_real* out = static_cast<io_real*>(a.observables_out);
+                for (int k = 0; k < Cfg::n_saved_obs; ++k)
+                    out[row_index<Cfg>(a, run, row, Cfg::n_saved_obs, k)] = io_real(0);
+            }
+            if constexpr (Cfg::save_counters) {
+                for (int k = 0; k < 4; ++k) a.counters_out[row_index<Cfg>(a, run, row, 4, k)] = 0;
+            }
+        }
+    }
+};
+
+// Row sink of adaptive runs in the plain kernel. The lanes of a wavefront
+// reach a save time at different loop iterations, so each lane puts its rows
+// into a ring of R row slots in LDS (lane index fastest: no bank conflicts at
+// whatever slot a lane is), and the wavefront writes row `base` of the
+// (time, variable, run) layout with one full-width store per column once
+// every lane has passed it. A lane R rows ahead of `base` waits; the lane at
+// `base` never does, so the wavefront always moves on, and it has to wait for
+// its slowest lane anyway.
+//
+// What bounds an output-heavy launch is HBM: this form writes each byte once
+// and whole lines at a time, where staging run-major wrote 1.6 times the
+// bytes (lines leave L2 partly filled), read and wrote them again in a
+// transpose, and needed the staging cleared first. Lorenz, 131,072 runs, 251
+// rows of state and time, FP64: 592 + 485 + 165 us before, 465 us now (1.05 GB
+// of rows, 0.21 ms at the copy rate); 250,003 runs, 161 rows, FP32: 442 + 507
+// + 80 -> 337 us. Two slots do as well as eight there; 16 cost occupancy
+// (675 us).
+template <typename Cfg>
+struct RowRing {
+    using io_real = typename Cfg::io_real;
+    static constexpr int R = Cfg::row_ring;   // a power of two
+    static constexpr int W = Cfg::n_saved_states + (Cfg::save_time ? 1 : 0);
+    static constexpr int NO = Cfg::save_obs ? Cfg::n_saved_obs : 0;
+    static constexpr int V = W + NO;                       // real values per row
+    static constexpr int C = Cfg::save_counters ? 4 : 0;   // counters per row
+    static constexpr int lanes = 64;
+    // LDS elements of one wavefront
+    static constexpr int vals_per_wave = R * V * lanes;
+    static constexpr int counts_per_wave = R * C * lanes;
+
+    io_real* vals;      // this lane's column of its wavefront's [R][V][64]
+    int* counts;        // and of [R][C][64]
+    long long base;     // rows below it are in the output; the same in every lane
+    long long left;     // rows from `base` to the last
+    long long limit;    // a lane that has saved this many rows waits
+    io_real* state_row;      // this lane's place in row `base` of each output
+    io_real* obs_row;
+    int* counts_row;
+
+    __device__ __forceinline__ void bind(const cubie_solve_args& a, long long run, io_real* v,
+                                         int* c) {
+        const int wave = threadIdx.x / lanes, lane = threadIdx.x % lanes;
+        vals = v + wave * vals_per_wave + lane;
+        counts = c + wave * counts_per_wave + lane;
+        state_row = static_cast<io_real*>(a.state_out) + run;
+        obs_row = static_cast<io_real*>(a.observables_out) + run;
+        counts_row = a.counters_out + run;
+        base = 0;
+        left = a.out_rows > 0 ? a.out_rows : 0;
+        set_limit();
+    }
+    // R rows ahead of `base` there is no slot; rows past the last are not kept
+    __device__ __forceinline__ void set_limit() {
+        limit = left > R ? base + R : 0x7fffffffffffffffLL;
+    }
+
+    template <typename S, typename O>
+    __device__ __forceinline__ void save(const cubie_solve_args& a, long long /*run*/, long long row,
+                                         const S& state, const O& obs, const int* cnt,
+                                         typename Cfg::real t_prec) {
+        if (row >= a.out_rows) return;
+        const int slot = int(row) & (R - 1);
+        io_real* v = vals + slot * (V * lanes);
+CUBIE_UNROLL
+        for (int k = 0; k < Cfg::n_saved_states; ++k)
+            v[k * lanes] = io_real(state[Cfg::saved_state_idx[k]]);
+        if constexpr (Cfg::save_time) v[Cfg::n_saved_states * lanes] = io_real(t_prec);
+CUBIE_UNROLL
+        for (int k = 0; k < NO; ++k) v[(W + k) * lanes] = io_real(obs[Cfg::saved_obs_idx[k]]);
+        if constexpr (C > 0) {
+            int* n = counts + slot * (C * lanes);
+CUBIE_UNROLL
+            for (int k = 0; k < C; ++k) n[k * lanes] = cnt[k];
+        }
+    }
+
+    // Write every row all lanes have passed; a finished lane's missing rows
+    // read zero. Called by all lanes of the wavefront that hold a run. Most
+    // calls find nothing to write: the places in the outputs are carried from
+    // row to row, so that such a call costs one vote.
+    __device__ __forceinline__ void flush(const cubie_solve_args& a, long long save_idx,
+                                          bool done) {
+        const long long passed = done ? 0x7fffffffffffffffLL : save_idx;
+        if (left == 0 || !wave_all(passed > base)) return;
+        const long long N = a.n_runs;
+        do {
+            const int slot = int(base) & (R - 1);
+            const io_real* v = vals + slot * (V * lanes);
+            const int* n = counts + slot * (C * lanes);
+            if (wave_all(save_idx > base)) {
+                if constexpr (W > 0) {
+CUBIE_UNROLL
+                    for (int k = 0; k < W; ++k) state_row[k * N] = v[k * lanes];
+                }
+CUBIE_UNROLL
+                for (int k = 0; k < NO; ++k) obs_row[k * N] = v[(W + k) * lanes];
+CUBIE_UNROLL
+                for (int k = 0; k < C; ++k) counts_row[k * N] = n[k * lanes];
+            } else {
+                const bool have = save_idx > base;
+                for (int k = 0; k < W; ++k) state_row[k * N] = have ? v[k * lanes] : io_real(0);
+                for (int k = 0; k < NO; ++k)
+                    obs_row[k * N] = have ? v[(W + k) * lanes] : io_real(0);
+                for (int k = 0; k < C; ++k) counts_row[k * N] = have ? n[k * lanes] : 0;
+            }
+            state_row += W * N;
+            obs_row += NO * N;
+            counts_row += C * N;
+            base += 1;
+            left -= 1;
+        } while (left != 0 && wave_all(passed > base));
+        set_limit();
+    }
+    __device__ __forceinline__ void zero_tail(const cubie_solve_args&, long long, long long) const {}
+};
 
 }  // namespace cubie

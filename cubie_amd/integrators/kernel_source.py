@@ -159,6 +159,9 @@ class KernelSpec:
     # per-row outputs staged run-major (run, time, variable); the host
     # transposes them to the (time, variable, run) layout after the launch
     run_major_rows: bool = False
+    # rows of LDS each lane of the plain kernel buffers its saves in (0: none;
+    # RowRing in outputs.hpp)
+    row_ring: int = 0
 
     # -- helpers ---------------------------------------------------------------
     @property
@@ -189,10 +192,13 @@ class KernelSpec:
         """Buffer placement of this kernel: ``buffer_placement``, or for
         "auto" registers up to PLACEMENT_REGISTER_MAX_N states and the
         private segment (HBM) beyond."""
-        if self.buffer_placement != "auto":
-            return self.buffer_placement
-        n = self.system.num_states
-        return "registers" if n <= self.PLACEMENT_REGISTER_MAX_N else "memory"
+        return self.placement_of(self.buffer_placement, self.system.num_states)
+
+    @classmethod
+    def placement_of(cls, buffer_placement: str, n: int) -> str:
+        if buffer_placement != "auto":
+            return buffer_placement
+        return "registers" if n <= cls.PLACEMENT_REGISTER_MAX_N else "memory"
 
     @property
     def sparse_jac_enabled(self) -> bool:
@@ -338,6 +344,8 @@ class KernelSpec:
         # (cuda_simsafe.py:171-188, adaptive_PI_controller.py:171)
         a(f"  static constexpr bool fast_controller = {str(not self.deterministic_pow).lower()};")
         a(f"  static constexpr bool run_major_rows = {str(bool(self.run_major_rows)).lower()};")
+        a(f"  static constexpr int row_ring = {int(self.row_ring)};")
+        a(f"  static constexpr int block_size = {int(self.block_size)};")
         # controller
         a(f"  static constexpr int controller = {ctrl.id};")
         a(f"  static constexpr real atol[{max(n, 1)}] = {c_array(ctrl.atol, wp)};")
