@@ -53,6 +53,14 @@ def _compile_only() -> bool:
     return os.environ.get("CUBIE_COMPILE_ONLY", "") == "1"
 
 
+def _compute_units() -> int:
+    """Compute units of the current device (a full MI355X without one)."""
+    import torch
+    if not torch.cuda.is_available():
+        return 256
+    return torch.cuda.get_device_properties(torch.device("cuda")).multi_processor_count
+
+
 def _torch():
     import torch
     if not torch.cuda.is_available():
@@ -64,6 +72,9 @@ def _torch():
 # operation; at relative tolerances below this floor it is of the order of the
 # error estimate itself, so the compensated mode hands such runs to FP64
 COMPENSATED_RTOL_FLOOR = 1e-6
+KERNEL_NAMES = {"plain": "cubie_integrate", "persistent": "cubie_integrate_persistent",
+                "record": "cubie_integrate_record", "adjoint": "cubie_adjoint"}
+SIMDS_PER_CU = 4
 # LDS of the row ring: bytes per lane, and per workgroup at most
 ROW_RING_LANE = 160
 ROW_RING_LDS = 80 * 1024
@@ -376,18 +387,20 @@ class BatchSolverKernel:
 
     def spec_for(self, duration: float, per_run_rtol: bool = False, adjoint: bool = False,
                  adj_ckpt_every: int = 32, block_size: Optional[int] = None,
-                 kernel_mode: Optional[str] = None) -> KernelSpec:
-        """The kernel specification for one run; ``block_size`` (default: the
-        configured one) is compiled into the kernel's launch bounds, and the
-        way rows are written follows ``kernel_mode`` (default: the configured
-        one)."""
+                 kernel_mode: Optional[str] = None,
+                 waves_per_eu: Optional[int] = None) -> KernelSpec:
+        """The kernel specification for one run; ``block_size`` and
+        ``waves_per_eu`` (default: the configured ones) are compiled into the
+        kernel's launch bounds, and the way rows are written follows
+        ``kernel_mode`` (default: the configured one)."""
         timing = self.timing.with_duration(duration)
+        waves_per_eu = self.waves_per_eu if waves_per_eu is None else int(waves_per_eu)
         block_size = int(block_size or self.block_size)
         staged = self.run_major_rows(adjoint, kernel_mode, block_size)
         ring = self.row_ring(adjoint, kernel_mode, block_size)
         key = (timing.summarise_every, timing.sample_summaries_every, per_run_rtol,
                self.precision_mode, self.fp_contract, block_size, self.deterministic_pow,
-               self.waves_per_eu, bool(adjoint), int(adj_ckpt_every), self.compensated_rhs,
+               waves_per_eu, bool(adjoint), int(adj_ckpt_every), self.compensated_rhs,
                self.buffer_placement, staged, ring, self.compensated_stage_rhs,
                self.sparse_jacobian, self.compensated_jacobian)
         if key not in self._spec_cache:
@@ -397,7 +410,7 @@ class BatchSolverKernel:
                 drivers=self.driver_interpolator, implicit=self.implicit,
                 compensated=self.precision_mode == "compensated", per_run_rtol=per_run_rtol,
                 fp_contract=self.fp_contract, block_size=block_size,
-                deterministic_pow=self.deterministic_pow, waves_per_eu=self.waves_per_eu,
+                deterministic_pow=self.deterministic_pow, waves_per_eu=waves_per_eu,
                 adjoint=bool(adjoint), adj_ckpt_every=int(adj_ckpt_every),
                 compensated_rhs=self.compensated_rhs, buffer_placement=self.buffer_placement,
                 run_major_rows=staged, row_ring=ring,
@@ -405,6 +418,34 @@ class BatchSolverKernel:
                 sparse_jacobian=self.sparse_jacobian,
                 compensated_jacobian=self.compensated_jacobian)
         return self._spec_cache[key]
+
+    def launch_spec(self, n_runs: int, duration: float, per_run_rtol: bool = False,
+                    block_size: Optional[int] = None,
+                    kernel_mode: Optional[str] = None) -> KernelSpec:
+        """``spec_for`` with the occupancy this batch asks for.
+
+        A kernel of 257 to 512 VGPRs runs one wavefront per SIMD. With more
+        wavefronts in the batch than SIMDs, the rest wait for a whole second
+        round, and no other wavefront fills the gaps between a wavefront's
+        dependent FP64 instructions; held to 256 VGPRs (a floor of two
+        wavefronts per SIMD) it spills a few values and runs two. Measured on
+        Hodgkin-Huxley SDIRK3 in FP64 (301 VGPRs; 184 bytes of spills a lane
+        with the floor), 12.5 ms at 2^-6: 65,536 runs 10.7 ms without and 12.0
+        with the floor, 131,072 runs 21.3 and 18.4, 262,144 runs 42.3 and 35.1;
+        65,600 runs, one wavefront too many, 80.9 and 67.0 over 50 ms. Batches of at most
+        one wavefront per SIMD keep the compiler's own choice, as does a
+        configured ``waves_per_eu``."""
+        spec = self.spec_for(duration, per_run_rtol, block_size=block_size,
+                             kernel_mode=kernel_mode)
+        if spec.waves_per_eu or math.ceil(n_runs / 64) <= SIMDS_PER_CU * _compute_units():
+            return spec
+        mode = kernel_mode or self.kernel_mode
+        regs = kcache.vgprs_of_parts(spec.source_parts(), spec.compile_options(),
+                                     KERNEL_NAMES[mode])
+        if regs is None or not 256 < regs <= 512:
+            return spec
+        return self.spec_for(duration, per_run_rtol, block_size=block_size,
+                             kernel_mode=kernel_mode, waves_per_eu=2)
 
     def config_key(self, duration: float, per_run_rtol: bool = False) -> str:
         """Digest of everything that fixes the kernel's work except the launch
@@ -422,9 +463,8 @@ class BatchSolverKernel:
 
     def module(self, spec: KernelSpec, kernel_mode: Optional[str] = None):
         mode = kernel_mode or self.kernel_mode
-        name = {"plain": "cubie_integrate", "persistent": "cubie_integrate_persistent",
-                "record": "cubie_integrate_record", "adjoint": "cubie_adjoint"}[mode]
-        return kcache.get_module_of_parts(spec.source_parts(), spec.compile_options(), name)
+        return kcache.get_module_of_parts(spec.source_parts(), spec.compile_options(),
+                                          KERNEL_NAMES[mode])
 
     def compile_only(self, duration: float = 1.0, per_run_rtol: bool = False) -> bytes:
         """Compile (or fetch from the cache) without touching a GPU."""
@@ -455,8 +495,9 @@ class BatchSolverKernel:
         """
         if _compile_only():
             dur = float(np.float64(duration))
-            spec = self.spec_for(dur, rtol_per_run is not None, block_size=blocksize,
-                                 kernel_mode=kernel_mode)
+            n = int(inits.shape[1]) if len(inits.shape) == 2 else 1
+            spec = self.launch_spec(n, dur, rtol_per_run is not None, block_size=blocksize,
+                                    kernel_mode=kernel_mode)
             kcache.get_code(spec.source(), spec.compile_options())
             if self._fp64_fallback_runs(inits, rtol_per_run) is not None:
                 twin = self.fp64_twin().spec_for(dur, rtol_per_run is not None,
@@ -484,15 +525,15 @@ class BatchSolverKernel:
         st = self.setup(inits, params, duration, warmup, t0, rtol_per_run, duration_per_run,
                         work_tally=work_tally, kernel_mode=mode, block_size=blocksize)
         # a requested block size is compiled into the kernel's launch bounds
-        spec = self.spec_for(st["duration"], st["per_run_rtol"], block_size=blocksize,
-                             kernel_mode=mode)
+        spec = self.launch_spec(st["n_runs"], st["duration"], st["per_run_rtol"],
+                                block_size=blocksize, kernel_mode=mode)
         mod = self.module(spec, mode)
         n_runs, args = st["n_runs"], st["args"]
         block = spec.block_size
         if mode == "plain":
             grid = max(1, math.ceil(n_runs / block))
         else:
-            cus = torch.cuda.get_device_properties(torch.device("cuda")).multi_processor_count
+            cus = _compute_units()
             grid = max(1, min(math.ceil(n_runs / block), cus * self.blocks_per_cu))
         stream = torch.cuda.current_stream().cuda_stream
         ms = None
@@ -903,13 +944,13 @@ class BatchSolverKernel:
             st = self.setup(inits[:, :m], params[:, :m] if params.size else params, duration,
                             warmup, t0, sl(rtol, 0, m), sl(dpr, 0, m), rows_duration=rows_dur,
                             kernel_mode=mode)
-            spec = self.spec_for(st["duration"], st["per_run_rtol"], kernel_mode=mode)
+            spec = self.launch_spec(m, st["duration"], st["per_run_rtol"], kernel_mode=mode)
             mod = self.module(spec, mode)
             block = spec.block_size
             if mode == "plain":
                 grid = max(1, math.ceil(m / block))
             else:
-                cus = torch.cuda.get_device_properties(torch.device("cuda")).multi_processor_count
+                cus = _compute_units()
                 grid = max(1, min(math.ceil(m / block), cus * self.blocks_per_cu))
             ins = [("inits", st["inits"])]
             if st["params"].numel() and params.size:

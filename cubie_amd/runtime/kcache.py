@@ -13,9 +13,10 @@ from __future__ import annotations
 
 import hashlib
 import os
+import re
 import tempfile
 import threading
-from typing import Dict, List, Tuple
+from typing import Dict, List, Optional, Tuple
 
 from . import native
 
@@ -29,6 +30,7 @@ _modules: Dict[Tuple[str, str], "native.Module"] = {}
 # spares joining and hashing the whole text on each launch
 _by_parts: Dict[tuple, "native.Module"] = {}
 PARTS_KEPT = 256
+_vgprs: Dict[tuple, Optional[int]] = {}
 _parts_lock = threading.Lock()
 
 
@@ -75,6 +77,19 @@ def get_module(source: str, options: List[str], kernel: str) -> "native.Module":
     return _modules[mk]
 
 
+def vgprs_of_parts(parts: Tuple[str, ...], options: List[str], kernel: str) -> Optional[int]:
+    """``vgpr_count`` of the kernel in the translation unit the pieces make."""
+    pk = (parts, tuple(options), kernel)
+    if pk not in _vgprs:
+        regs = vgpr_count(get_code("\n".join(parts), options)[1], kernel)
+        with _parts_lock:
+            while len(_vgprs) >= PARTS_KEPT:
+                del _vgprs[next(iter(_vgprs))]
+            _vgprs[pk] = regs
+        return regs
+    return _vgprs[pk]
+
+
 def get_module_of_parts(parts: Tuple[str, ...], options: List[str],
                         kernel: str) -> "native.Module":
     """``get_module`` of the translation unit the pieces make."""
@@ -87,3 +102,17 @@ def get_module_of_parts(parts: Tuple[str, ...], options: List[str],
                 del _by_parts[next(iter(_by_parts))]
             _by_parts[pk] = mod
     return mod
+
+
+def vgpr_count(code: bytes, kernel: str) -> Optional[int]:
+    """Vector registers per lane of one kernel, from the code object's own
+    metadata (a msgpack map whose keys are sorted: ``.symbol``, the kernel's
+    name and ".kd", precedes ``.vgpr_count``); None if it is not found. Needs
+    no device."""
+    m = re.search(rb"\.symbol(?:[\xa0-\xbf]|\xd9.)" + re.escape(kernel.encode())
+                  + rb"\.kd(?:(?!\.symbol).)*?\.vgpr_count(\xcd..|\xcc.|[\x00-\x7f])",
+                  code, re.DOTALL)
+    if m is None:
+        return None
+    raw = m.group(1)
+    return raw[0] if len(raw) == 1 else int.from_bytes(raw[1:], "big")
