@@ -62,6 +62,16 @@ __device__ __forceinline__ bool dfinite(float x) { return __builtin_isfinite(x);
 __device__ __forceinline__ double dfloor(double x) { return __builtin_floor(x); }
 __device__ __forceinline__ float dfloor(float x) { return __builtin_floorf(x); }
 
+// x, kept out of a fused multiply-add: a product passed through here is
+// rounded before it is added.
+template <typename T>
+__device__ __forceinline__ T rounded(T x) {
+#ifdef __AMDGCN__
+    asm("" : "+v"(x));
+#endif
+    return x;
+}
+
 // Wavefront-wide vote over the currently active lanes, the wave64
 // counterpart of the reference's all_sync(activemask(), pred)
 // (cuda_simsafe.py:610).

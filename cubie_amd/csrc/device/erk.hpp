@@ -21,7 +21,9 @@ struct ERKStep {
     static constexpr int s = Cfg::stages;
     Vec<real, n> stage_rhs;   // persistent: FSAL cache
     // In the compensated mode: the step's increment y_{n+1} - y_n before it
-    // is rounded into y, for the loop's Kahan-compensated state update.
+    // is rounded into y, for the loop's Kahan-compensated state update. It is
+    // a rounded product there in every kernel (not fused into that update in
+    // some), so that the plain and the persistent kernel agree bit for bit.
     Vec<real, (Cfg::kahan_state ? n : 1)> increment;
 
     __device__ __forceinline__ void init() {
@@ -72,7 +74,7 @@ CUBIE_UNROLL
             if constexpr (Cfg::kahan_state && Cfg::b_row >= 0) {
                 if (prev == Cfg::b_row - 1) {
 CUBIE_UNROLL
-                    for (int i = 0; i < n; ++i) increment[i] = acc[prev * n + i] * dt;
+                    for (int i = 0; i < n; ++i) increment[i] = rounded(acc[prev * n + i] * dt);
                 }
             }
 CUBIE_UNROLL
@@ -103,7 +105,7 @@ CUBIE_UNROLL
         }
 CUBIE_UNROLL
         for (int i = 0; i < n; ++i) {
-            if constexpr (Cfg::kahan_state && Cfg::accumulates_output) increment[i] = proposed[i] * dt;
+            if constexpr (Cfg::kahan_state && Cfg::accumulates_output) increment[i] = rounded(proposed[i] * dt);
             if constexpr (Cfg::accumulates_output) proposed[i] = proposed[i] * dt + state[i];
             if constexpr (Cfg::has_error) {
                 if constexpr (Cfg::accumulates_error) error[i] *= dt;
