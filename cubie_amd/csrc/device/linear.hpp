@@ -50,6 +50,7 @@ struct SolverConsts;
 template <>
 struct SolverConsts<double> {
     static constexpr double clamp = 1e150;
+    static constexpr double product_safe = 1e75;
     static constexpr double breakdown = 1e-200;
     static constexpr double huge = 1.7976931348623157e308;
     static constexpr double stagnation_eps = 1.4901161193847656e-06;  // 100*sqrt(eps)
@@ -57,6 +58,7 @@ struct SolverConsts<double> {
 template <>
 struct SolverConsts<float> {
     static constexpr float clamp = 1e16f;
+    static constexpr float product_safe = 1e8f;
     static constexpr float breakdown = 1e-30f;
     static constexpr float huge = 3.4028234663852886e38f;
     static constexpr float stagnation_eps = 0.034526698300124390f;      // 100*sqrt(eps)
@@ -202,10 +204,111 @@ CUBIE_UNROLL
     return converged ? ST_SUCCESS : ST_LINEAR_MAX_ITERS;
 }
 
+// The running maximum of |x| the clamp tests below are made with. A NaN drops
+// out of it: the clamps leave NaNs alone.
+template <typename T>
+__device__ __forceinline__ T max_abs(T m, T x) {
+    if constexpr (same_type<T, double>::value) return __builtin_fmax(m, dabs(x));
+    else return __builtin_fmaxf(m, dabs(x));
+}
+
+// A product in one of BiCGSTAB's sums. Guarded FP32 solves round it before
+// they add it, as clamping it does: with the products fused, one FP32
+// Robertson run of 64 stopped short of its stopping test, which is within an
+// order of magnitude of FP32's resolution.
+template <typename Cfg, typename T>
+__device__ __forceinline__ T kprod(T a, T b) {
+    if constexpr (!Cfg::krylov_fast && same_type<T, float>::value) return rounded(a * b);
+    else return a * b;
+}
+
+// The pieces of one BiCGSTAB iteration. With Careful every value is clamped
+// as the reference clamps it, before the next use; without, nothing is
+// clamped and `m` collects the largest magnitude. When that is at most
+// SolverConsts::product_safe (the square root of the clamp), neither a vector
+// entry nor a product of two can have reached the clamp, and both forms give
+// the same values.
+template <typename Cfg, bool Careful, typename L, typename Prob>
+__device__ __forceinline__ void bicgstab_direction(const Prob& P, const L* p, const L* r0_hat,
+                                                   L* tmp, L* v, L& dot_r0v, L& m) {
+    constexpr int W = Prob::W;
+    precondition<Cfg, L>(P, p, tmp);
+    if constexpr (Careful) {
+CUBIE_UNROLL
+        for (int i = 0; i < W; ++i) tmp[i] = clampc(tmp[i]);
+    }
+    P.op(tmp, v);
+    dot_r0v = L(0);
+CUBIE_UNROLL
+    for (int i = 0; i < W; ++i) {
+        if constexpr (Careful) {
+            v[i] = clampc(v[i]);
+            dot_r0v += clampc(r0_hat[i] * v[i]);
+        } else {
+            dot_r0v += kprod<Cfg>(r0_hat[i], v[i]);
+            m = max_abs(max_abs(m, tmp[i]), v[i]);
+        }
+    }
+}
+
+template <typename Cfg, bool Careful, typename L, typename Prob>
+__device__ __forceinline__ void bicgstab_smoothing(const Prob& P, const L* rhs, L* s_hat, L* tmp,
+                                                   L& dot_ts, L& dot_tt, L& m) {
+    constexpr int W = Prob::W;
+    precondition<Cfg, L>(P, rhs, s_hat);
+    if constexpr (Careful) {
+CUBIE_UNROLL
+        for (int i = 0; i < W; ++i) s_hat[i] = clampc(s_hat[i]);
+    }
+    P.op(s_hat, tmp);
+    dot_ts = L(0);
+    dot_tt = L(0);
+CUBIE_UNROLL
+    for (int i = 0; i < W; ++i) {
+        if constexpr (Careful) {
+            const L ti = clampc(tmp[i]);
+            tmp[i] = ti;
+            dot_ts += clampc(ti * rhs[i]);
+            dot_tt += clamp_pos(ti * ti);
+        } else {
+            dot_ts += kprod<Cfg>(tmp[i], rhs[i]);
+            dot_tt += kprod<Cfg>(tmp[i], tmp[i]);
+            m = max_abs(max_abs(max_abs(m, s_hat[i]), tmp[i]), rhs[i]);
+        }
+    }
+}
+
+template <typename Cfg, bool Careful, int W, typename L>
+__device__ __forceinline__ L bicgstab_rho(const L* r0_hat, const L* rhs, L& m) {
+    L rho = L(0);
+CUBIE_UNROLL
+    for (int i = 0; i < W; ++i) {
+        if constexpr (Careful) {
+            rho += clampc(r0_hat[i] * rhs[i]);
+        } else {
+            rho += kprod<Cfg>(r0_hat[i], rhs[i]);
+            m = max_abs(m, rhs[i]);
+        }
+    }
+    return rho;
+}
+
 // Preconditioned BiCGSTAB with the reference's clamps and breakdown guards.
+//
+// VALU-issue bound, in FP64 mostly by the clamps when each is made where the
+// reference makes it: two compares and four selects a value, 27 values an
+// iteration for three states, more than half of its instructions. Here one
+// maximum a value and one compare a piece tell whether any clamp could act;
+// only then the piece is done again with its clamps. A lane that has
+// converged (or broken down) at the half step leaves there: the second half
+// changes nothing for it. Before -> after: Robertson ROS3P, 20,001 runs to 1e4,
+// 94.0 -> 65.5 ms; Radau IIA, 30,000 runs to 1e3, 21.7 -> 14.2 ms; Hodgkin-Huxley
+// SDIRK3 FP64, 65,600 runs over 50 ms, 67.0 -> 53.4 ms.
 template <typename Cfg, typename L, typename Prob>
 __device__ __forceinline__ int bicgstab_solve(Prob& P, L* rhs, L* x, bool x_is_zero, int& iters) {
     constexpr int W = Prob::W;
+    constexpr bool guarded = !Cfg::krylov_fast;   // the clamps apply (kclamp)
+    constexpr L safe = SolverConsts<L>::product_safe;
     constexpr L brk = SolverConsts<L>::breakdown;
     constexpr L dclamp = SolverConsts<L>::clamp;
     const L rhs_norm2 = P.krylov_norm2(rhs);
@@ -219,6 +322,7 @@ CUBIE_UNROLL
         for (int i = 0; i < W; ++i) tmp[i] = L(0);
     }
     L rho_prev = L(0);
+    L m0 = L(0);          // |r0_hat| enters every product with it
 CUBIE_UNROLL
     for (int i = 0; i < W; ++i) {
         const L ax = kclamp<Cfg>(tmp[i]);
@@ -227,6 +331,7 @@ CUBIE_UNROLL
         r0_hat[i] = ri;
         p[i] = kclamp<Cfg>(ri);
         rho_prev += kclamp_pos<Cfg>(ri * ri);
+        if constexpr (guarded) m0 = max_abs(m0, ri);
     }
     L acc = P.krylov_norm2(rhs);
     bool converged = acc <= tol2;
@@ -236,69 +341,68 @@ CUBIE_UNROLL
     for (int k = 0; k < Cfg::krylov_max_iters; ++k) {
         if (finished) break;
         ++it;
-        precondition<Cfg, L>(P, p, tmp);
-CUBIE_UNROLL
-        for (int i = 0; i < W; ++i) tmp[i] = kclamp<Cfg>(tmp[i]);
-        P.op(tmp, v);
-        L dot_r0v = L(0);
-CUBIE_UNROLL
-        for (int i = 0; i < W; ++i) {
-            v[i] = kclamp<Cfg>(v[i]);
-            dot_r0v += kclamp<Cfg>(r0_hat[i] * v[i]);
+        L m = m0;
+        L dot_r0v;
+        bicgstab_direction<Cfg, false>(P, p, r0_hat, tmp, v, dot_r0v, m);
+        if constexpr (guarded) {
+            if (m > safe) bicgstab_direction<Cfg, true>(P, p, r0_hat, tmp, v, dot_r0v, m);
         }
         const bool alpha_overflow = dabs(rho_prev) > dabs(dot_r0v) * dclamp;
-        broken = broken || (!finished && alpha_overflow);
-        finished = converged || broken;
+        broken = broken || alpha_overflow;
         const L alpha = (dot_r0v != L(0) && !alpha_overflow) ? kdiv<Cfg>(rho_prev, dot_r0v) : L(0);
-        const L alpha_eff = finished ? L(0) : alpha;
+        const L alpha_eff = broken ? L(0) : alpha;
 CUBIE_UNROLL
         for (int i = 0; i < W; ++i) {
             x[i] = x[i] + alpha_eff * tmp[i];
             rhs[i] = rhs[i] - alpha_eff * v[i];
         }
         acc = P.krylov_norm2(rhs);
-        converged = converged || (acc <= tol2);
+        converged = acc <= tol2;
         finished = converged || broken;
-        precondition<Cfg, L>(P, rhs, s_hat);
-CUBIE_UNROLL
-        for (int i = 0; i < W; ++i) s_hat[i] = kclamp<Cfg>(s_hat[i]);
-        P.op(s_hat, tmp);
-        L dot_ts = L(0), dot_tt = L(0);
-CUBIE_UNROLL
-        for (int i = 0; i < W; ++i) {
-            const L ti = kclamp<Cfg>(tmp[i]);
-            tmp[i] = ti;
-            dot_ts += kclamp<Cfg>(ti * rhs[i]);
-            dot_tt += kclamp_pos<Cfg>(ti * ti);
+        if (finished) break;
+        m = m0;
+        L dot_ts, dot_tt;
+        bicgstab_smoothing<Cfg, false>(P, rhs, s_hat, tmp, dot_ts, dot_tt, m);
+        if constexpr (guarded) {
+            if (m > safe) bicgstab_smoothing<Cfg, true>(P, rhs, s_hat, tmp, dot_ts, dot_tt, m);
         }
         const bool omega_overflow = dabs(dot_ts) > dot_tt * dclamp;
         const L omega = (dot_tt != L(0) && !omega_overflow) ? kdiv<Cfg>(dot_ts, dot_tt) : L(0);
-        const L omega_eff = finished ? L(0) : omega;
 CUBIE_UNROLL
         for (int i = 0; i < W; ++i) {
-            x[i] = x[i] + omega_eff * s_hat[i];
-            rhs[i] = rhs[i] - omega_eff * tmp[i];
+            x[i] = x[i] + omega * s_hat[i];
+            rhs[i] = rhs[i] - omega * tmp[i];
         }
         acc = P.krylov_norm2(rhs);
-        converged = converged || (acc <= tol2);
-        L rho_new = L(0);
-CUBIE_UNROLL
-        for (int i = 0; i < W; ++i) rho_new += kclamp<Cfg>(r0_hat[i] * rhs[i]);
+        converged = acc <= tol2;
+        m = m0;
+        L rho_new = bicgstab_rho<Cfg, false, W>(r0_hat, rhs, m);
+        if constexpr (guarded) {
+            if (m > safe) rho_new = bicgstab_rho<Cfg, true, W>(r0_hat, rhs, m);
+        }
         const bool rho_bad = dabs(rho_new) < brk;
         const bool omega_bad = dabs(omega) < brk;
-        broken = broken || (!converged && (rho_bad || omega_bad));
+        broken = !converged && (rho_bad || omega_bad);
         finished = converged || broken;
         const bool beta_overflow = (dabs(rho_new) > dabs(rho_prev) * dclamp) ||
                                    (dabs(alpha) > dabs(omega) * dclamp);
         broken = broken || (!finished && beta_overflow);
         finished = converged || broken;
-        const L beta = !finished ? kdiv<Cfg>(rho_new, rho_prev) * kdiv<Cfg>(alpha, omega) : L(0);
+        if (finished) break;
+        const L beta = kdiv<Cfg>(rho_new, rho_prev) * kdiv<Cfg>(alpha, omega);
+        m = L(0);
 CUBIE_UNROLL
         for (int i = 0; i < W; ++i) {
-            L pi = !finished ? rhs[i] + beta * (p[i] - omega * v[i]) : p[i];
-            p[i] = kclamp<Cfg>(pi);
+            p[i] = rhs[i] + beta * (p[i] - omega * v[i]);
+            if constexpr (guarded) m = max_abs(m, p[i]);
         }
-        rho_prev = !finished ? rho_new : rho_prev;
+        if constexpr (guarded) {
+            if (m > dclamp) {
+CUBIE_UNROLL
+                for (int i = 0; i < W; ++i) p[i] = clampc(p[i]);
+            }
+        }
+        rho_prev = rho_new;
     }
     iters = it;
     return converged ? ST_SUCCESS : (broken ? ST_BICGSTAB_BREAKDOWN : ST_LINEAR_MAX_ITERS);

@@ -1,0 +1,62 @@
+"""BiCGSTAB near and beyond its value clamps, on the CPU: the kernel skips the
+clamps of a piece of an iteration when no value of it is large enough to meet
+them. Against the host build that always makes them, states from ordinary to
+far past the clamps (1e16 in FP32, 1e150 in FP64, and their square roots, where
+products meet them) give the same statuses, counters and states."""
+
+import numpy as np
+import pytest
+
+import cubie_amd as ca
+import host_build
+from cubie_amd.integrators.kernel_source import KernelSpec
+from systems import lorenz, lorenz_batch, robertson, robertson_batch
+
+ALWAYS = {"product_safe = 1e75": "product_safe = -1.0", "product_safe = 1e8f":
+          "product_safe = -1.0f"}
+
+
+def _both(monkeypatch, solver, inits, params, duration):
+    source = KernelSpec.source
+    out = [host_build.solve(solver, inits, params, duration)]
+
+    def careful(self):
+        text = source(self)
+        for old, new in ALWAYS.items():
+            assert old in text
+            text = text.replace(old, new)
+        return text
+
+    with monkeypatch.context() as m:
+        m.setattr(KernelSpec, "source", careful)
+        out.append(host_build.solve(solver, inits, params, duration))
+    for k in ("status_codes", "iteration_counters", "state", "work_tally"):
+        assert np.array_equal(out[0][k], out[1][k], equal_nan=out[0][k].dtype.kind == "f"), k
+    return out[0]
+
+
+@pytest.mark.parametrize("algorithm", ["backwards_euler", "l_stable_dirk_3", "radau", "ros3p"])
+@pytest.mark.parametrize("precision,scales", [
+    (np.float32, [1.0, 1e3, 3e4, 1e7, 1e8, 3e8, 1e12, 1e15, 1e30]),
+    (np.float64, [1.0, 1e20, 1e37, 1e60, 1e75, 1e80, 1e120, 1e149, 1e250])])
+def test_states_across_the_clamps(monkeypatch, algorithm, precision, scales):
+    base, params = lorenz_batch(4, seed=31)
+    inits = np.concatenate([base * s for s in scales], axis=1).astype(precision)
+    params = np.tile(params, (1, len(scales))).astype(precision)
+    # a step at which ordinary states converge, and one that keeps h times the
+    # quadratic terms small for many of the large ones
+    for dt in (2.0 ** -10, 2.0 ** -60):
+        solver = ca.Solver(lorenz(precision), algorithm=algorithm, dt=dt, atol=1e-6, rtol=1e-4,
+                           step_controller="fixed", linear_correction_type="bicgstab",
+                           krylov_max_iters=20, newton_max_iters=20, save_every=4 * dt,
+                           output_types=["state", "iteration_counters"], deterministic_pow=True)
+        _both(monkeypatch, solver, inits, params, 8 * dt)
+
+
+def test_stiff_adaptive_runs(monkeypatch):
+    inits, params = robertson_batch(6, seed=32)
+    solver = ca.Solver(robertson(np.float64), algorithm="ros3p", atol=1e-10, rtol=1e-6,
+                       linear_correction_type="bicgstab", save_every=10.0,
+                       output_types=["state", "iteration_counters"], deterministic_pow=True)
+    out = _both(monkeypatch, solver, inits, params, 100.0)
+    assert np.all(out["status_codes"] == 0)
