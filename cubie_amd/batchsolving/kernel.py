@@ -435,17 +435,29 @@ class BatchSolverKernel:
         65,600 runs, one wavefront too many, 80.9 and 67.0 over 50 ms. Batches of at most
         one wavefront per SIMD keep the compiler's own choice, as does a
         configured ``waves_per_eu``."""
+        return self._launch_parts(n_runs, duration, per_run_rtol, block_size, kernel_mode)[0]
+
+    def _launch_parts(self, n_runs, duration, per_run_rtol, block_size, kernel_mode):
+        """``launch_spec`` and the pieces of its translation unit, made once."""
         spec = self.spec_for(duration, per_run_rtol, block_size=block_size,
                              kernel_mode=kernel_mode)
+        parts = spec.source_parts()
         if spec.waves_per_eu or math.ceil(n_runs / 64) <= SIMDS_PER_CU * _compute_units():
-            return spec
+            return spec, parts
         mode = kernel_mode or self.kernel_mode
-        regs = kcache.vgprs_of_parts(spec.source_parts(), spec.compile_options(),
-                                     KERNEL_NAMES[mode])
+        regs = kcache.vgprs_of_parts(parts, spec.compile_options(), KERNEL_NAMES[mode])
         if regs is None or not 256 < regs <= 512:
-            return spec
-        return self.spec_for(duration, per_run_rtol, block_size=block_size,
+            return spec, parts
+        spec = self.spec_for(duration, per_run_rtol, block_size=block_size,
                              kernel_mode=kernel_mode, waves_per_eu=2)
+        return spec, spec.source_parts()
+
+    def launch_module(self, n_runs: int, duration: float, per_run_rtol: bool = False,
+                      block_size: Optional[int] = None, kernel_mode: Optional[str] = None):
+        """``launch_spec`` and its loaded module."""
+        spec, parts = self._launch_parts(n_runs, duration, per_run_rtol, block_size, kernel_mode)
+        mode = kernel_mode or self.kernel_mode
+        return spec, kcache.get_module_of_parts(parts, spec.compile_options(), KERNEL_NAMES[mode])
 
     def config_key(self, duration: float, per_run_rtol: bool = False) -> str:
         """Digest of everything that fixes the kernel's work except the launch
@@ -525,9 +537,8 @@ class BatchSolverKernel:
         st = self.setup(inits, params, duration, warmup, t0, rtol_per_run, duration_per_run,
                         work_tally=work_tally, kernel_mode=mode, block_size=blocksize)
         # a requested block size is compiled into the kernel's launch bounds
-        spec = self.launch_spec(st["n_runs"], st["duration"], st["per_run_rtol"],
-                                block_size=blocksize, kernel_mode=mode)
-        mod = self.module(spec, mode)
+        spec, mod = self.launch_module(st["n_runs"], st["duration"], st["per_run_rtol"],
+                                       block_size=blocksize, kernel_mode=mode)
         n_runs, args = st["n_runs"], st["args"]
         block = spec.block_size
         if mode == "plain":
@@ -944,8 +955,8 @@ class BatchSolverKernel:
             st = self.setup(inits[:, :m], params[:, :m] if params.size else params, duration,
                             warmup, t0, sl(rtol, 0, m), sl(dpr, 0, m), rows_duration=rows_dur,
                             kernel_mode=mode)
-            spec = self.launch_spec(m, st["duration"], st["per_run_rtol"], kernel_mode=mode)
-            mod = self.module(spec, mode)
+            spec, mod = self.launch_module(m, st["duration"], st["per_run_rtol"],
+                                           kernel_mode=mode)
             block = spec.block_size
             if mode == "plain":
                 grid = max(1, math.ceil(m / block))
