@@ -18,10 +18,14 @@ Two kernels from one module (``cubie_amd/csrc/device/adjoint.hpp``):
 
 HBM per system: (sizeof(real) + 1) bytes per accepted step of tape,
 (n + 1) values per checkpoint, and replay buffers of
-(K + 1) (n + 1) + K s n values (K = checkpoint_every, s = stages). Tape length
-is the largest accepted-step count of the batch: when ``max_steps`` is not
-given a counting pass (the recording kernel with an empty tape) measures it
-first.
+(K + 1) (n + 1) + K s n values (K = checkpoint_every, s = stages). With
+``checkpoint_every`` left at its default and the memory for it (half of what
+is free), every step is a checkpoint: the backward pass then replays nothing.
+Tape length is the largest accepted-step count of the batch. When
+``max_steps`` is not given, the first recording goes into a tape of bounded
+size (TAPE_FIRST_TRY); its step counts are right in any case, so if it was too
+short (or too little fits it to try) one more pass records into a tape of the
+counted length.
 
 The reference has no adjoint; this module is an extension of the engine.
 """
@@ -38,6 +42,11 @@ from ..runtime import kcache, native
 from ..result_codes import CUBIE_RESULT_CODES
 from .kernel import CompileOnly, _compile_only
 
+DEFAULT_CHECKPOINT_EVERY = 32
+# bytes of the first recording's tape when the step count is not known, and
+# the fewest steps worth trying it for
+TAPE_FIRST_TRY = 16 << 30
+FIRST_TRY_STEPS = 64
 # summary metrics whose gradient the backward pass propagates
 DIFFERENTIABLE_METRICS = {"mean", "rms", "max", "min"}
 
@@ -66,7 +75,7 @@ def _grid(n_runs: int, block: int) -> int:
 
 def record(kernel, inits, params, duration: float, warmup: float = 0.0, t0: float = 0.0,
            rtol_per_run=None, duration_per_run=None, max_steps: Optional[int] = None,
-           checkpoint_every: int = 32, timed: bool = False) -> AdjointRecord:
+           checkpoint_every: int = DEFAULT_CHECKPOINT_EVERY, timed: bool = False) -> AdjointRecord:
     """Forward solve that records the adjoint's tape; returns the record
     (outputs under ``record.outputs``)."""
     if checkpoint_every < 1:
@@ -76,54 +85,98 @@ def record(kernel, inits, params, duration: float, warmup: float = 0.0, t0: floa
     import torch
     st = kernel.setup(inits, params, duration, warmup, t0, rtol_per_run, duration_per_run,
                       adjoint=True)
-    spec = kernel.spec_for(st["duration"], st["per_run_rtol"], adjoint=True,
-                           adj_ckpt_every=checkpoint_every)
-    mod = kernel.module(spec, "record")
     dev = torch.device("cuda")
     n_runs = st["n_runs"]
     n = kernel.system.num_states
     tdt = torch.float32 if kernel.precision is np.float32 else torch.float64
-    block = spec.block_size
     stream = torch.cuda.current_stream().cuda_stream
 
-    def launch(max_st: int, max_ck: int, timed_: bool):
+    def launch(every: int, rows: int, timed_: bool):
+        """Record with checkpoints every ``every`` steps into ``rows`` steps
+        of tape."""
+        spec = kernel.spec_for(st["duration"], st["per_run_rtol"], adjoint=True,
+                               adj_ckpt_every=every)
+        block = spec.block_size
+        n_ck = rows // every + 1
         bufs = {
-            "tape_dt": torch.empty((max(max_st, 1), n_runs), dtype=tdt, device=dev),
-            "tape_flags": torch.empty((max(max_st, 1), n_runs), dtype=torch.uint8, device=dev),
-            "checkpoints": torch.empty((max(max_ck, 1), n, n_runs), dtype=tdt, device=dev),
-            "checkpoint_t": torch.empty((max(max_ck, 1), n_runs), dtype=torch.float64, device=dev),
-            "tape_info": torch.zeros((3, n_runs), dtype=torch.int32, device=dev),
+            "tape_dt": torch.empty((max(rows, 1), n_runs), dtype=tdt, device=dev),
+            "tape_flags": torch.empty((max(rows, 1), n_runs), dtype=torch.uint8, device=dev),
+            "checkpoints": torch.empty((n_ck, n, n_runs), dtype=tdt, device=dev),
+            "checkpoint_t": torch.empty((n_ck, n_runs), dtype=torch.float64, device=dev),
+            "tape_info": torch.empty((3, n_runs), dtype=torch.int32, device=dev),
         }
-        a = native.AdjointArgs()
-        a.fwd = st["args"]
-        a.checkpoints = bufs["checkpoints"].data_ptr()
-        a.checkpoint_t = bufs["checkpoint_t"].data_ptr()
-        a.tape_dt = bufs["tape_dt"].data_ptr()
-        a.tape_flags = bufs["tape_flags"].data_ptr()
-        a.tape_info = bufs["tape_info"].data_ptr()
-        a.max_steps = int(max_st)
-        a.max_checkpoints = int(max_ck)
-        ms = mod.launch_adjoint(a, _grid(n_runs, block), block, stream, timed=timed_)
-        return a, bufs, ms
+        a = _tape_args(st, bufs, rows, n_ck)
+        ms = kernel.module(spec, "record").launch_adjoint(a, _grid(n_runs, block), block, stream,
+                                                          timed=timed_)
+        return AdjointRecord(kernel=kernel, spec=spec, setup=st, args=a, buffers=bufs,
+                             max_steps=rows, max_checkpoints=n_ck, checkpoint_every=every,
+                             record_ms=ms)
 
+    def counted(rec: AdjointRecord) -> int:
+        return int(rec.buffers["tape_info"][0].max().item()) if n_runs else 0
+
+    every_step = checkpoint_every == DEFAULT_CHECKPOINT_EVERY
+    # state, step size, time and flags of one step of the whole batch
+    step_bytes = (torch.finfo(tdt).bits // 8 * (n + 1) + 9) * max(n_runs, 1)
+    available = _available_bytes(torch) if every_step else 0
+    if max_steps is None and every_step:
+        rows = int(min(TAPE_FIRST_TRY, available // 16) // step_bytes) - 1
+        if rows >= FIRST_TRY_STEPS:
+            rec = launch(1, rows, timed)
+            max_steps = counted(rec)
+            if max_steps <= rows:
+                _trim(rec, max_steps)
+                return rec
+            del rec
     if max_steps is None:
         # counting pass: an empty tape, the kernel still counts the steps
-        _, cbufs, _ = launch(0, 0, False)
-        max_steps = int(cbufs["tape_info"][0].max().item()) if n_runs else 0
-        st["outputs"].status_codes.zero_()
+        max_steps = counted(launch(1 if every_step else checkpoint_every, 0, False))
     max_steps = int(max_steps)
-    max_ck = max_steps // checkpoint_every + 1
-    args, bufs, ms = launch(max_steps, max_ck, timed)
-    return AdjointRecord(kernel=kernel, spec=spec, setup=st, args=args, buffers=bufs,
-                         max_steps=max_steps, max_checkpoints=max_ck,
-                         checkpoint_every=checkpoint_every, record_ms=ms)
+    if every_step and step_bytes * (max_steps + 1) <= available // 2:
+        return launch(1, max_steps, timed)
+    return launch(checkpoint_every, max_steps, timed)
+
+
+def _available_bytes(torch) -> int:
+    """Device memory a new tensor could take: free, or cached by torch."""
+    free, _total = torch.cuda.mem_get_info()
+    return int(free + torch.cuda.memory_reserved() - torch.cuda.memory_allocated())
+
+
+def _tape_args(st, bufs, rows: int, n_ck: int):
+    a = native.AdjointArgs()
+    a.fwd = st["args"]
+    a.checkpoints = bufs["checkpoints"].data_ptr()
+    a.checkpoint_t = bufs["checkpoint_t"].data_ptr()
+    a.tape_dt = bufs["tape_dt"].data_ptr()
+    a.tape_flags = bufs["tape_flags"].data_ptr()
+    a.tape_info = bufs["tape_info"].data_ptr()
+    a.max_steps = int(rows)
+    a.max_checkpoints = int(n_ck)
+    return a
+
+
+def _trim(rec: AdjointRecord, steps: int) -> None:
+    """A tape with a checkpoint at every step, cut to the steps it holds when
+    those are less than half of it (the copy is two passes over them)."""
+    if 2 * steps < rec.max_steps:
+        b = rec.buffers
+        for key in ("tape_dt", "tape_flags"):
+            b[key] = b[key][:max(steps, 1)].clone()
+        for key in ("checkpoints", "checkpoint_t"):
+            b[key] = b[key][:steps + 1].clone()
+        rec.max_checkpoints = steps + 1
+        rec.args = _tape_args(rec.setup, b, steps, steps + 1)
+    rec.max_steps = steps
 
 
 def _compile(kernel, duration, per_run_rtol, checkpoint_every):
     """CUBIE_COMPILE_ONLY=1: cache the adjoint module and stop."""
-    spec = kernel.spec_for(float(np.float64(duration)), per_run_rtol, adjoint=True,
-                           adj_ckpt_every=checkpoint_every)
-    kcache.get_code(spec.source(), spec.compile_options())
+    for every in {checkpoint_every, 1} if checkpoint_every == DEFAULT_CHECKPOINT_EVERY else {
+            checkpoint_every}:
+        spec = kernel.spec_for(float(np.float64(duration)), per_run_rtol, adjoint=True,
+                               adj_ckpt_every=every)
+        kcache.get_code(spec.source(), spec.compile_options())
     raise CompileOnly(spec)
 
 
@@ -184,19 +237,19 @@ def backward(rec: AdjointRecord, grad_state=None, grad_state_summaries=None,
     gss = grad_like(grad_state_summaries, outs.state_summaries)
     _check_summary_grads(kernel, gss)
     bufs = {
-        "replay": torch.empty((K + 1, n, n_runs), dtype=tdt, device=dev),
-        "replay_t": torch.empty((K + 1, n_runs), dtype=torch.float64, device=dev),
-        "replay_stages": torch.empty((K, S, n_runs), dtype=tdt, device=dev),
-        "grad_inits": torch.zeros((n, n_runs), dtype=tdt, device=dev),
-        "grad_params": torch.zeros((max(npar, 1), n_runs), dtype=tdt, device=dev),
+        "grad_inits": torch.empty((n, n_runs), dtype=tdt, device=dev),
+        "grad_params": torch.empty((max(npar, 1), n_runs), dtype=tdt, device=dev),
     }
+    if K > 1:
+        bufs["replay"] = torch.empty((K + 1, n, n_runs), dtype=tdt, device=dev)
+        bufs["replay_t"] = torch.empty((K + 1, n_runs), dtype=torch.float64, device=dev)
+        bufs["replay_stages"] = torch.empty((K, S, n_runs), dtype=tdt, device=dev)
     a = native.AdjointArgs()
     a.fwd = st["args"]
     for k in ("checkpoints", "checkpoint_t", "tape_dt", "tape_flags", "tape_info"):
         setattr(a, k, getattr(rec.args, k))
-    a.replay = bufs["replay"].data_ptr()
-    a.replay_t = bufs["replay_t"].data_ptr()
-    a.replay_stages = bufs["replay_stages"].data_ptr()
+    for k in ("replay", "replay_t", "replay_stages"):
+        setattr(a, k, bufs[k].data_ptr() if k in bufs else 0)
     a.grad_state = gs.data_ptr() if gs is not None else 0
     a.grad_state_summ = gss.data_ptr() if gss is not None else 0
     a.grad_inits = bufs["grad_inits"].data_ptr()
@@ -222,9 +275,15 @@ def _function():
         def forward(ctx, inits, params, kernel, duration, opts):
             rec = record(kernel, inits.detach(), params.detach(), duration, **opts)
             ctx.rec = rec
+            # new tensor objects over the same memory: returning the record's
+            # own would tie the graph's node, the record and these outputs
+            # into a reference cycle, and the tape would live until the
+            # garbage collector came by
             out = rec.outputs
-            ctx.mark_non_differentiable(out.status_codes)
-            return out.state, out.state_summaries, out.status_codes
+            state, summaries, status = (out.state.detach(), out.state_summaries.detach(),
+                                        out.status_codes.detach())
+            ctx.mark_non_differentiable(status)
+            return state, summaries, status
 
         @staticmethod
         def backward(ctx, g_state, g_summ, _g_status):
@@ -238,7 +297,8 @@ _FN = None
 
 
 def solve_adjoint(solver, inits, params, duration: float, warmup: float = 0.0, t0: float = 0.0,
-                  max_steps: Optional[int] = None, checkpoint_every: int = 32,
+                  max_steps: Optional[int] = None,
+                  checkpoint_every: int = DEFAULT_CHECKPOINT_EVERY,
                   rtol_per_run=None, duration_per_run=None):
     """Differentiable batch solve: returns torch tensors ``(state,
     state_summaries, status)`` laid out like the solver's device outputs

@@ -18,6 +18,17 @@
 // step. Replay buffers: [K+1][n][N] states, [K+1][N] times, [K][stash][N]
 // stage values, with the run axis fastest (coalesced across a wave).
 //
+// With a checkpoint at every step (Cfg::adj_ckpt_every == 1, which the host
+// chooses where the memory allows it) there is nothing to replay: each step's
+// stages are formed from its own start state just before its adjoint and stay
+// in registers (whole_step). On Hodgkin-Huxley (DOPRI5, six parameters) the
+// replay moved 0.58 KB a step through HBM and evaluated the right-hand side's
+// exponentials twice, once for the stages and once in the vector-Jacobian
+// products; whole_step reads 49 bytes a step and, where the stage Jacobians
+// fit in registers (adjoint_keeps_jacobians), evaluates them once. Backward
+// pass over 25 ms, before -> after: DOPRI5, 100,000 runs, 12.7 -> 5.4 ms (20 GB
+// of HBM traffic -> 2.6); ROS3P, 40,001 runs, 22 -> 12.9 ms (27 GB -> 5).
+//
 // One step's adjoint, lambda = dL/dy_{k+1} in, dL/dy_k out:
 //   explicit RK: y+ = y + h sum_i b_i k_i, k_i = f(Y_i), Y_i = y + h sum_j a_ij k_j
 //     g_i = h b_i lambda + h sum_{j>i} a_ji w_j,  w_i = J(Y_i)^T g_i,
@@ -38,6 +49,61 @@
 namespace cubie {
 
 // DenseLU (partial pivoting, in registers) is defined with the linear solvers.
+
+// Stages that feed the solution, or a later stage that does.
+template <int s>
+struct LiveStages {
+    bool v[s] = {};
+    int count = 0;
+};
+template <typename Cfg>
+__device__ constexpr LiveStages<Cfg::stages> live_stages() {
+    LiveStages<Cfg::stages> l;
+    for (int i = Cfg::stages - 1; i >= 0; --i) {
+        bool live = Cfg::b[i] != 0.0;
+        for (int j = i + 1; j < Cfg::stages; ++j) live = live || (l.v[j] && Cfg::A[j][i] != 0.0);
+        l.v[i] = live;
+        l.count += live ? 1 : 0;
+    }
+    return l;
+}
+
+// Whether whole_step holds every live stage's Jacobian: `per_stage` values of
+// J and about 2 n of stage vectors a stage, within 320 of a lane's 512 VGPRs.
+template <typename Cfg, typename Sys>
+__device__ constexpr bool adjoint_keeps_jacobians(int live) {
+    return Cfg::n * Cfg::n <= 64 &&
+           live * (Sys::jac_nnz + 2 * Cfg::n) * int(sizeof(typename Cfg::real) / 4) <= 320;
+}
+
+// gy = J^T w and mu += f_p^T w at one stage, J given.
+template <typename Cfg, typename Sys, typename Ctx>
+__device__ __forceinline__ void stage_vjp(Ctx& ctx, const typename Cfg::real* Y,
+                                          const typename Cfg::real* J,
+                                          const typename Cfg::real* w, typename Cfg::real* gy,
+                                          typename Cfg::real* mu, typename Cfg::real ts) {
+    using real = typename Cfg::real;
+    constexpr int n = Cfg::n;
+    constexpr int P = Cfg::n_params;
+CUBIE_UNROLL
+    for (int j = 0; j < n; ++j) {
+        real acc = real(0);
+CUBIE_UNROLL
+        for (int i = 0; i < n; ++i)
+            if (Sys::jac_nz[i * n + j]) acc += J[i * n + j] * w[i];
+        gy[j] = acc;
+    }
+    if constexpr (P > 0) {
+        real Jp[n * P];
+        Sys::jacp(Y, ctx.params.data(), ctx.proposed_drivers.data(), Jp, ts);
+CUBIE_UNROLL
+        for (int q = 0; q < P; ++q) {
+CUBIE_UNROLL
+            for (int i = 0; i < n; ++i)
+                if (Sys::jacp_nz[i * P + q]) mu[q] += Jp[i * P + q] * w[i];
+        }
+    }
+}
 
 // ---------------------------------------------------------------------------
 // Explicit Runge-Kutta step adjoint
@@ -98,6 +164,55 @@ CUBIE_UNROLL
             for (int i = 0; i < s; ++i)
                 if (Cfg::b[i] != 0.0) acc += Cfg::b[i] * kst[i * n + c];
             y[c] = acc * h + y[c];
+        }
+    }
+
+    static constexpr LiveStages<s> alive = live_stages<Cfg>();
+    static constexpr bool keep_jac = adjoint_keeps_jacobians<Cfg, Sys>(alive.count);
+
+    // One step from its start state alone: the stages, then their adjoints.
+    template <typename Ctx>
+    __device__ __forceinline__ static void whole_step(Ctx& ctx, const real* y, real t, real h,
+                                                      real* lam, real* mu) {
+        real kst[s * n];
+        if constexpr (!keep_jac) {
+            real yy[n];
+CUBIE_UNROLL
+            for (int c = 0; c < n; ++c) yy[c] = y[c];
+            replay(ctx, yy, t, h, kst);
+            backward(ctx, y, t, h, kst, lam, mu);
+        } else {
+            real J[s][n * n], G[s * n];
+CUBIE_UNROLL
+            for (int i = 0; i < s; ++i) {
+                if (!alive.v[i]) continue;
+                real Y[n], obs[Cfg::n_obs > 0 ? Cfg::n_obs : 1];
+                stage_state(y, h, kst, i, Y);
+                const real ts = t + h * Cfg::c[i];
+                ctx.drv.eval(ts, ctx.proposed_drivers.data());
+                Sys::dxdt_jac(Y, ctx.params.data(), ctx.proposed_drivers.data(), obs, &kst[i * n],
+                              J[i], ts);
+CUBIE_UNROLL
+                for (int c = 0; c < n; ++c) G[i * n + c] = (h * Cfg::b[i]) * lam[c];
+            }
+CUBIE_UNROLL
+            for (int i = s - 1; i >= 0; --i) {
+                if (!alive.v[i]) continue;
+                real Y[n], w[n];
+                stage_state(y, h, kst, i, Y);
+                const real ts = t + h * Cfg::c[i];
+                ctx.drv.eval(ts, ctx.proposed_drivers.data());
+                stage_vjp<Cfg, Sys>(ctx, Y, J[i], &G[i * n], w, mu, ts);
+CUBIE_UNROLL
+                for (int c = 0; c < n; ++c) lam[c] += w[c];
+CUBIE_UNROLL
+                for (int j = 0; j < s; ++j) {
+                    if (j < i && alive.v[j] && Cfg::A[i][j] != 0.0) {
+CUBIE_UNROLL
+                        for (int c = 0; c < n; ++c) G[j * n + c] += (h * Cfg::A[i][j]) * w[c];
+                    }
+                }
+            }
         }
     }
 
@@ -186,11 +301,12 @@ CUBIE_UNROLL
         }
     }
 
-    template <typename Ctx>
-    __device__ __forceinline__ static void replay(Ctx& ctx, real* y, real t, real h, real* kst) {
-        DenseLU<real, n> lu;
-        real fdt[n], dd[nd > 0 ? nd : 1];
-        step_matrix(ctx, y, t, h, lu, fdt, dd);
+    // The stage increments kst, and with J a [s][n n] array (not nullptr_t)
+    // every stage's Jacobian.
+    template <typename Ctx, typename JS>
+    __device__ __forceinline__ static void stages(Ctx& ctx, const real* y, real t, real h,
+                                                  const DenseLU<real, n>& lu, const real* fdt,
+                                                  real* kst, JS&& J) {
         const real inv_h = real(1) / h;
 CUBIE_UNROLL
         for (int i = 0; i < s; ++i) {
@@ -198,7 +314,10 @@ CUBIE_UNROLL
             stage_state(y, kst, i, Y);
             const real ts = t + h * Cfg::c[i];
             ctx.drv.eval(ts, ctx.proposed_drivers.data());
-            Sys::dxdt(Y, ctx.params.data(), ctx.proposed_drivers.data(), obs, f, ts);
+            if constexpr (same_type<JS, decltype(nullptr)>::value)
+                Sys::dxdt(Y, ctx.params.data(), ctx.proposed_drivers.data(), obs, f, ts);
+            else
+                Sys::dxdt_jac(Y, ctx.params.data(), ctx.proposed_drivers.data(), obs, f, J[i], ts);
 CUBIE_UNROLL
             for (int c = 0; c < n; ++c) {
                 real corr = real(0);
@@ -210,6 +329,14 @@ CUBIE_UNROLL
             }
             lu.solve(&kst[i * n]);
         }
+    }
+
+    template <typename Ctx>
+    __device__ __forceinline__ static void replay(Ctx& ctx, real* y, real t, real h, real* kst) {
+        DenseLU<real, n> lu;
+        real fdt[n], dd[nd > 0 ? nd : 1];
+        step_matrix(ctx, y, t, h, lu, fdt, dd);
+        stages(ctx, y, t, h, lu, fdt, kst, nullptr);
 CUBIE_UNROLL
         for (int c = 0; c < n; ++c) {
             real v = y[c];
@@ -220,12 +347,40 @@ CUBIE_UNROLL
         }
     }
 
+    static constexpr bool keep_jac = adjoint_keeps_jacobians<Cfg, Sys>(s);
+
+    // One step from its start state alone: W = I - gamma h J(y_n) is formed
+    // and factored once for the stages and their adjoints.
+    template <typename Ctx>
+    __device__ __forceinline__ static void whole_step(Ctx& ctx, const real* y, real t, real h,
+                                                      real* lam, real* mu) {
+        DenseLU<real, n> lu;
+        real fdt[n], dd[nd > 0 ? nd : 1], kst[s * n];
+        step_matrix(ctx, y, t, h, lu, fdt, dd);
+        if constexpr (keep_jac) {
+            real J[s][n * n];
+            stages(ctx, y, t, h, lu, fdt, kst, J);
+            adjoints(ctx, y, t, h, lu, dd, kst, J, lam, mu);
+        } else {
+            stages(ctx, y, t, h, lu, fdt, kst, nullptr);
+            adjoints(ctx, y, t, h, lu, dd, kst, nullptr, lam, mu);
+        }
+    }
+
     template <typename Ctx>
     __device__ __forceinline__ static void backward(Ctx& ctx, const real* y, real t, real h,
                                                     const real* kst, real* lam, real* mu) {
         DenseLU<real, n> lu;
         real fdt[n], dd[nd > 0 ? nd : 1];
         step_matrix(ctx, y, t, h, lu, fdt, dd);
+        adjoints(ctx, y, t, h, lu, dd, kst, nullptr, lam, mu);
+    }
+
+    // The stages' adjoints, last to first; J as in stages().
+    template <typename Ctx, typename JS>
+    __device__ __forceinline__ static void adjoints(Ctx& ctx, const real* y, real t, real h,
+                                                    const DenseLU<real, n>& lu, const real* dd,
+                                                    const real* kst, JS&& J, real* lam, real* mu) {
         real Kb[s * n];
 CUBIE_UNROLL
         for (int i = 0; i < s; ++i)
@@ -245,11 +400,15 @@ CUBIE_UNROLL
             ctx.drv.eval(ts, ctx.proposed_drivers.data());
 CUBIE_UNROLL
             for (int c = 0; c < n; ++c) wz[c] = gh * z[c];
-            Sys::vjp(Y, ctx.params.data(), ctx.proposed_drivers.data(), wz, w, wp, ts);
+            if constexpr (same_type<JS, decltype(nullptr)>::value) {
+                Sys::vjp(Y, ctx.params.data(), ctx.proposed_drivers.data(), wz, w, wp, ts);
+CUBIE_UNROLL
+                for (int q = 0; q < P; ++q) mu[q] += wp[q];
+            } else {
+                stage_vjp<Cfg, Sys>(ctx, Y, J[i], wz, w, mu, ts);
+            }
 CUBIE_UNROLL
             for (int c = 0; c < n; ++c) lam[c] += w[c];
-CUBIE_UNROLL
-            for (int q = 0; q < P; ++q) mu[q] += wp[q];
 CUBIE_UNROLL
             for (int j = 0; j < s; ++j) {
                 if (j < i) {
@@ -379,6 +538,96 @@ CUBIE_UNROLL
     }
 }
 
+// Largest value over the lanes of a full wavefront.
+__device__ __forceinline__ int wave_max(int x) {
+    for (int off = 32; off > 0; off >>= 1) {
+        const int o = __shfl_xor(x, off);
+        x = o > x ? o : x;
+    }
+    return x;
+}
+
+// Backward pass over a tape with the state and time of every step. The lanes
+// of a wavefront go through the step index together (lanes whose run took
+// fewer steps join later), so its reads are whole lines; the next step's
+// values are read while this one is worked on.
+template <typename Cfg, typename Sys, typename Adj>
+__device__ __forceinline__ void adjoint_backward_every_step(const cubie_adjoint_args& A) {
+    using real = typename Cfg::real;
+    using io_real = typename Cfg::io_real;
+    constexpr int n = Cfg::n;
+    constexpr int P = Cfg::n_params;
+    const cubie_solve_args& a = A.fwd;
+    const long long N = a.n_runs;
+    const long long lane_run = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const bool valid = lane_run < N;
+    const long long run = valid ? lane_run : 0;   // every lane stays for the votes
+
+    LoopCtx<Cfg> ctx;
+    ctx.drv.coeffs = static_cast<const io_real*>(a.driver_coeffs);
+    const io_real* params = static_cast<const io_real*>(a.params);
+CUBIE_UNROLL
+    for (int q = 0; q < P; ++q) ctx.params[q] = real(params[q * N + run]);
+    real lam[n], mu[P > 0 ? P : 1];
+CUBIE_UNROLL
+    for (int c = 0; c < n; ++c) lam[c] = real(0);
+CUBIE_UNROLL
+    for (int q = 0; q < (P > 0 ? P : 1); ++q) mu[q] = real(0);
+
+    const int steps = valid ? A.tape_info[run] : 0;
+    long long save_i = valid ? A.tape_info[N + run] : 0;
+    long long upd_i = valid ? A.tape_info[2 * N + run] : 0;
+    const real* tdt = static_cast<const real*>(A.tape_dt);
+    const real* ck = static_cast<const real*>(A.checkpoints);
+    unsigned found = 0u;
+    long long window = -1;
+
+    struct Step {
+        real y[n], h;
+        double t;
+        unsigned flags;
+    };
+    const auto read = [&](long long j, Step& s) {
+        if (j >= 0 && j < steps) {
+CUBIE_UNROLL
+            for (int c = 0; c < n; ++c) s.y[c] = ck[(j * n + c) * N + run];
+            s.t = A.checkpoint_t[j * N + run];
+            s.h = tdt[j * N + run];
+            s.flags = A.tape_flags[j * N + run];
+        }
+    };
+    Step cur = {}, nxt = {};
+    const int top = wave_max(steps);
+    read(top - 1, cur);
+    for (int j = top - 1; j >= 0; --j) {
+        read(j - 1, nxt);
+        if (j < steps) {
+            if (cur.flags) {
+                real y_end[n];
+CUBIE_UNROLL
+                for (int c = 0; c < n; ++c) y_end[c] = ck[((long long)(j + 1) * n + c) * N + run];
+                add_output_grads<Cfg>(A, run, cur.flags, save_i, upd_i, found, window, y_end, lam);
+            }
+            Adj::whole_step(ctx, cur.y, real(cur.t), cur.h, lam, mu);
+        }
+        cur = nxt;
+    }
+    if (!valid) return;
+    // the save row written at t0 (no settling time)
+    if (a.warmup == 0.0 && save_i > 0) {
+        real y0[n];
+CUBIE_UNROLL
+        for (int c = 0; c < n; ++c) y0[c] = ck[c * N + run];
+        add_output_grads<Cfg>(A, run, 1u, save_i, upd_i, found, window, y0, lam);
+    }
+    io_real* gi = static_cast<io_real*>(A.grad_inits);
+    io_real* gp = static_cast<io_real*>(A.grad_params);
+CUBIE_UNROLL
+    for (int c = 0; c < n; ++c) gi[c * N + run] = io_real(lam[c]);
+CUBIE_UNROLL
+    for (int q = 0; q < P; ++q) gp[q * N + run] = io_real(mu[q]);
+}
+
 // Backward pass: gradients of the loss with respect to inits and params.
 template <typename Cfg, typename Sys, typename Adj>
 __device__ __forceinline__ void adjoint_backward(const cubie_adjoint_args& A) {
@@ -388,6 +637,10 @@ __device__ __forceinline__ void adjoint_backward(const cubie_adjoint_args& A) {
     constexpr int P = Cfg::n_params;
     constexpr int S = Adj::stash;
     constexpr int K = Cfg::adj_ckpt_every;
+    if constexpr (K == 1) {
+        adjoint_backward_every_step<Cfg, Sys, Adj>(A);
+        return;
+    }
     const cubie_solve_args& a = A.fwd;
     const long long run = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (run >= a.n_runs) return;

@@ -686,6 +686,8 @@ class SystemCodegen:
         parts.append("    (void)y; (void)p; (void)d; (void)Jp; (void)t;")
         parts.append("  }")
         if self.adjoint:
+            nzp = ", ".join("true" if not e.is_zero else "false" for _, e in Jp)
+            parts.append(f"  static constexpr bool jacp_nz[{max(n * npar, 1)}] = {{{nzp or 'false'}}};")
             parts += self._emit_adjoint(dx, dfdt, dds)
         parts.append("};")
         return "\n".join(parts) + "\n"
