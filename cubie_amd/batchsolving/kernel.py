@@ -362,7 +362,9 @@ class BatchSolverKernel:
         0.16 ms), while lanes that wait for one another are not (60 ms)."""
         if (kernel_mode or self.kernel_mode) != "plain" or not self._rows_out_of_step(adjoint):
             return 0
-        if KernelSpec.placement_of(self.buffer_placement, self.system.num_states) != "registers":
+        if KernelSpec.placement_of(self.buffer_placement, self.system, self.algorithm,
+                                   self.precision, self.output_config,
+                                   self.precision_mode == "compensated") != "registers":
             return 0
         oc = self.output_config
         item = np.dtype(self.precision).itemsize
@@ -432,8 +434,13 @@ class BatchSolverKernel:
         Hodgkin-Huxley SDIRK3 in FP64 (301 VGPRs; 184 bytes of spills a lane
         with the floor), 12.5 ms at 2^-6: 65,536 runs 10.7 ms without and 12.0
         with the floor, 131,072 runs 21.3 and 18.4, 262,144 runs 42.3 and 35.1;
-        65,600 runs, one wavefront too many, 80.9 and 67.0 over 50 ms. Batches of at most
-        one wavefront per SIMD keep the compiler's own choice, as does a
+        65,600 runs, one wavefront too many, 80.9 and 67.0 over 50 ms; Radau
+        IIA on Robertson (319 VGPRs, 248 bytes), 262,144 runs 17.3 and 15.4 ms.
+        Their spills lie outside the Krylov loops. An explicit step is one
+        straight line through all its values, and its spills cost more than
+        the second wavefront gives (DOPRI5 on 20 states, 333 VGPRs, 131,072
+        runs: 1.15 and 1.74 ms), so explicit kernels keep the compiler's own
+        choice, as do batches of at most one wavefront per SIMD and a
         configured ``waves_per_eu``."""
         return self._launch_parts(n_runs, duration, per_run_rtol, block_size, kernel_mode)[0]
 
@@ -442,7 +449,8 @@ class BatchSolverKernel:
         spec = self.spec_for(duration, per_run_rtol, block_size=block_size,
                              kernel_mode=kernel_mode)
         parts = spec.source_parts()
-        if spec.waves_per_eu or math.ceil(n_runs / 64) <= SIMDS_PER_CU * _compute_units():
+        if (spec.waves_per_eu or not self.algorithm.is_implicit
+                or math.ceil(n_runs / 64) <= SIMDS_PER_CU * _compute_units()):
             return spec, parts
         mode = kernel_mode or self.kernel_mode
         regs = kcache.vgprs_of_parts(parts, spec.compile_options(), KERNEL_NAMES[mode])

@@ -184,6 +184,9 @@ class KernelSpec:
     # state count above which "auto" keeps the per-system vectors in memory:
     # register-resident kernels of larger systems spill thousands of values
     PLACEMENT_REGISTER_MAX_N = 16
+    # 32-bit words of vectors an explicit kernel may hold beyond that (a lane
+    # has 512 VGPRs; the rest spills)
+    PLACEMENT_ERK_WORDS = 640
     # matrix-free problems hold the sparse Jacobian up to this many nonzeros
     SPARSE_JAC_MAX_NNZ = 4096
 
@@ -192,13 +195,45 @@ class KernelSpec:
         """Buffer placement of this kernel: ``buffer_placement``, or for
         "auto" registers up to PLACEMENT_REGISTER_MAX_N states and the
         private segment (HBM) beyond."""
-        return self.placement_of(self.buffer_placement, self.system.num_states)
+        if self.adjoint:
+            # the backward pass holds all stages and their adjoints at once
+            return self.placement_of(self.buffer_placement, self.system)
+        return self.placement_of(self.buffer_placement, self.system, self.algorithm,
+                                 self.precision, self.outputs, self.compensated)
 
     @classmethod
-    def placement_of(cls, buffer_placement: str, n: int) -> str:
+    def placement_of(cls, buffer_placement: str, system, algorithm=None, precision=None,
+                     outputs=None, compensated: bool = False) -> str:
+        """Placement of the per-system vectors (``resolved_placement``).
+
+        Explicit Runge-Kutta kernels (``algorithm`` given) hold the state, the
+        current derivative and one accumulator per stage still to come: about
+        stages + 1 vectors at a time, and the parameters, observables and
+        summary buffers. The unrolled form keeps them in registers well beyond
+        PLACEMENT_REGISTER_MAX_N states, where the loops' form moves every one
+        of them through the private segment several times a step. DOPRI5 in
+        FP64, Lorenz-96, 50,000 runs over one time unit, private segment
+        against registers: 20 states 21.2 and 0.38 ms, 32 states (503 VGPRs)
+        34.9 and 0.80 ms, 40 states (308 bytes spilled a lane) 44.0 and 2.3 ms,
+        48 states (752 bytes) 54.1 and 5.7 ms; 72 states in FP32 (416 bytes)
+        67.9 and 2.5 ms. The line is drawn at 40 and 80 states, where spills
+        start to grow faster than the states and compilation passes 20 s."""
         if buffer_placement != "auto":
             return buffer_placement
-        return "registers" if n <= cls.PLACEMENT_REGISTER_MAX_N else "memory"
+        n = system.num_states
+        if n <= cls.PLACEMENT_REGISTER_MAX_N:
+            return "registers"
+        if algorithm is None or algorithm.family != "erk":
+            return "memory"
+        held = ((algorithm.tableau.stage_count + 1 + (2 if compensated else 0)) * n
+                + system.num_parameters + 2 * (system.num_observables + system.num_drivers))
+        height = sum(summary_metrics[m].buffer_len(p) for m, p in outputs.metrics)
+        if outputs.summarise_state:
+            held += height * len(outputs.summarised_state_indices)
+        if outputs.summarise_observables:
+            held += height * len(outputs.summarised_observable_indices)
+        words = 2 if precision is np.float64 else 1
+        return "registers" if held * words <= cls.PLACEMENT_ERK_WORDS else "memory"
 
     @property
     def sparse_jac_enabled(self) -> bool:
