@@ -158,8 +158,8 @@ def _tape_args(st, bufs, rows: int, n_ck: int):
 
 def _trim(rec: AdjointRecord, steps: int) -> None:
     """A tape with a checkpoint at every step, cut to the steps it holds when
-    those are less than half of it (the copy is two passes over them)."""
-    if 2 * steps < rec.max_steps:
+    those are less than a quarter of it (the copy is two passes over them)."""
+    if 4 * steps < rec.max_steps:
         b = rec.buffers
         for key in ("tape_dt", "tape_flags"):
             b[key] = b[key][:max(steps, 1)].clone()

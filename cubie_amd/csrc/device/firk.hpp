@@ -90,7 +90,7 @@ CUBIE_UNROLL
 CUBIE_UNROLL
         for (int k = 0; k < n; ++k) {
             L tol = L(Cfg::krylov_atol[k]) + L(Cfg::krylov_rtol[k]) * dabs(L(base[k]));
-            kw[k] = L(1) / pmax(tol, L(1e-16));
+            kw[k] = sdiv<Cfg>(L(1), pmax(tol, L(1e-16)));
         }
     }
     // J(Y_i) dir for stage i
@@ -180,7 +180,7 @@ CUBIE_UNROLL
             const real ref = pmax(dabs(sv), dabs(base[k]));
             real tol = Cfg::newton_atol[k] + Cfg::newton_rtol[k] * ref;
             tol = pmax(tol, real(1e-16));
-            const real r = vals[e] / tol;
+            const real r = sdiv<Cfg>(vals[e], tol);
             nrm2 += r * r;
         }
         return nrm2 * real(1.0 / double(W));

@@ -77,6 +77,51 @@ __device__ __forceinline__ T clamp_pos(T x) {
     return x > c ? c : x;
 }
 
+// Quotients and square roots of the solvers' own scalars: tolerance weights,
+// Krylov coefficients, norms. Production builds take FP64 ones from the
+// hardware estimate (2^-23), one Newton step (2^-46) and a correction by the
+// exact residual: 7 instructions for a quotient that is the correctly rounded
+// one but for ties it comes within 2^-92 of, against 11 for the IEEE sequence,
+// whose scaling of extreme exponents costs the rest and a trip through VCC.
+// v_div_fixup puts in the IEEE results for zeros, infinities and NaNs. Without
+// the scaling a quotient of operands beyond about 1e+-290 may be off by 2^-46;
+// tolerances, and sums that the guards keep within the clamps, stay far from
+// there. Parity builds keep the IEEE operations, as the oracle has them.
+// With the clamps of a solve's start tested once and the maxima in chains of
+// their own: Robertson ROS3P 65.5 -> 58.5 ms, Radau 14.2 -> 13.3, Hodgkin-Huxley
+// SDIRK3 FP64 52.0 -> 45.9 (at the sizes given at bicgstab_solve).
+template <typename Cfg, typename T>
+__device__ __forceinline__ T sdiv(T a, T b) {
+#ifdef __AMDGCN__
+    if constexpr (Cfg::fast_controller && same_type<T, double>::value) {
+        double y = __builtin_amdgcn_rcp(b);
+        y = __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
+        double q = a * y;
+        q = __builtin_fma(__builtin_fma(-b, q, a), y, q);
+        return __builtin_amdgcn_div_fixup(q, b, a);
+    }
+#endif
+    return a / b;
+}
+// x >= 0 or NaN. The estimate of 1 / sqrt(x), refined once and corrected by
+// the residual x - g^2; zeros, infinities and NaNs are their own roots.
+template <typename Cfg, typename T>
+__device__ __forceinline__ T ssqrt(T x) {
+#ifdef __AMDGCN__
+    if constexpr (Cfg::fast_controller && same_type<T, double>::value) {
+        const double y = __builtin_amdgcn_rsq(x);
+        double g = x * y, h = 0.5 * y;
+        const double r = __builtin_fma(-h, g, 0.5);
+        g = __builtin_fma(g, r, g);
+        h = __builtin_fma(h, r, h);
+        g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+        // signalling and quiet NaN, +-0, +infinity
+        return __builtin_amdgcn_class(x, 0x263) ? x : g;
+    }
+#endif
+    return dsqrt(x);
+}
+
 // Krylov value clamps and divisions. The reference clamps every Krylov
 // vector and inner product to +-1e16 (FP32) / 1e150 (FP64) against overflow.
 // The compensated mode's FP32 solves (Cfg::krylov_fast) skip the clamps
@@ -85,19 +130,9 @@ __device__ __forceinline__ T clamp_pos(T x) {
 // production builds (Cfg::krylov_rcp) they also divide by the hardware
 // reciprocal, parity builds keep IEEE division.
 template <typename Cfg, typename T>
-__device__ __forceinline__ T kclamp(T x) {
-    if constexpr (Cfg::krylov_fast) return x;
-    else return clampc(x);
-}
-template <typename Cfg, typename T>
-__device__ __forceinline__ T kclamp_pos(T x) {
-    if constexpr (Cfg::krylov_fast) return x;
-    else return clamp_pos(x);
-}
-template <typename Cfg, typename T>
 __device__ __forceinline__ T kdiv(T a, T b) {
     if constexpr (Cfg::krylov_rcp && same_type<T, float>::value) return a * __builtin_amdgcn_rcpf(b);
-    else return a / b;
+    else return sdiv<Cfg>(a, b);
 }
 
 // Preconditioner application: the configured kinds in order (a single kind,
@@ -164,7 +199,7 @@ template <typename Cfg, typename L, typename Prob>
 __device__ __forceinline__ int mr_solve(Prob& P, L* rhs, L* x, bool x_is_zero, int& iters) {
     constexpr int W = Prob::W;
     const L rhs_norm2 = P.krylov_norm2(rhs);
-    const L tol = L(Cfg::krylov_floor) + L(Cfg::krylov_reduction) * L(dsqrt(rhs_norm2));
+    const L tol = L(Cfg::krylov_floor) + L(Cfg::krylov_reduction) * ssqrt<Cfg>(rhs_norm2);
     const L tol2 = tol * tol;
     L temp[W], z[W];
     if (!x_is_zero) {
@@ -239,6 +274,7 @@ CUBIE_UNROLL
     }
     P.op(tmp, v);
     dot_r0v = L(0);
+    [[maybe_unused]] L mv = L(0);   // a chain of its own, for the latency
 CUBIE_UNROLL
     for (int i = 0; i < W; ++i) {
         if constexpr (Careful) {
@@ -246,9 +282,11 @@ CUBIE_UNROLL
             dot_r0v += clampc(r0_hat[i] * v[i]);
         } else {
             dot_r0v += kprod<Cfg>(r0_hat[i], v[i]);
-            m = max_abs(max_abs(m, tmp[i]), v[i]);
+            m = max_abs(m, tmp[i]);
+            mv = max_abs(mv, v[i]);
         }
     }
+    if constexpr (!Careful) m = max_abs(m, mv);
 }
 
 template <typename Cfg, bool Careful, typename L, typename Prob>
@@ -263,6 +301,7 @@ CUBIE_UNROLL
     P.op(s_hat, tmp);
     dot_ts = L(0);
     dot_tt = L(0);
+    [[maybe_unused]] L mt = L(0), mr = L(0);
 CUBIE_UNROLL
     for (int i = 0; i < W; ++i) {
         if constexpr (Careful) {
@@ -273,9 +312,12 @@ CUBIE_UNROLL
         } else {
             dot_ts += kprod<Cfg>(tmp[i], rhs[i]);
             dot_tt += kprod<Cfg>(tmp[i], tmp[i]);
-            m = max_abs(max_abs(max_abs(m, s_hat[i]), tmp[i]), rhs[i]);
+            m = max_abs(m, s_hat[i]);
+            mt = max_abs(mt, tmp[i]);
+            mr = max_abs(mr, rhs[i]);
         }
     }
+    if constexpr (!Careful) m = max_abs(max_abs(m, mt), mr);
 }
 
 template <typename Cfg, bool Careful, int W, typename L>
@@ -303,16 +345,18 @@ CUBIE_UNROLL
 // converged (or broken down) at the half step leaves there: the second half
 // changes nothing for it. Before -> after: Robertson ROS3P, 20,001 runs to 1e4,
 // 94.0 -> 65.5 ms; Radau IIA, 30,000 runs to 1e3, 21.7 -> 14.2 ms; Hodgkin-Huxley
-// SDIRK3 FP64, 65,600 runs over 50 ms, 67.0 -> 53.4 ms.
+// SDIRK3 FP64, 65,600 runs over 50 ms, 67.0 -> 53.4 ms. (One test a solve, at
+// its end, with the solve done again where it fires, needs more registers and
+// scalar work: 68.4 ms where this form with the same quotients takes 60.9.)
 template <typename Cfg, typename L, typename Prob>
 __device__ __forceinline__ int bicgstab_solve(Prob& P, L* rhs, L* x, bool x_is_zero, int& iters) {
     constexpr int W = Prob::W;
-    constexpr bool guarded = !Cfg::krylov_fast;   // the clamps apply (kclamp)
+    constexpr bool guarded = !Cfg::krylov_fast;   // the clamps apply
     constexpr L safe = SolverConsts<L>::product_safe;
     constexpr L brk = SolverConsts<L>::breakdown;
     constexpr L dclamp = SolverConsts<L>::clamp;
     const L rhs_norm2 = P.krylov_norm2(rhs);
-    const L tol = L(Cfg::krylov_floor) + L(Cfg::krylov_reduction) * L(dsqrt(rhs_norm2));
+    const L tol = L(Cfg::krylov_floor) + L(Cfg::krylov_reduction) * ssqrt<Cfg>(rhs_norm2);
     const L tol2 = tol * tol;
     L r0_hat[W], p[W], v[W], tmp[W], s_hat[W];
     if (!x_is_zero) {
@@ -325,14 +369,27 @@ CUBIE_UNROLL
     L m0 = L(0);          // |r0_hat| enters every product with it
 CUBIE_UNROLL
     for (int i = 0; i < W; ++i) {
-        const L ax = kclamp<Cfg>(tmp[i]);
-        const L ri = rhs[i] - ax;
-        rhs[i] = ri;
-        r0_hat[i] = ri;
-        p[i] = kclamp<Cfg>(ri);
-        rho_prev += kclamp_pos<Cfg>(ri * ri);
-        if constexpr (guarded) m0 = max_abs(m0, ri);
+        r0_hat[i] = rhs[i] - tmp[i];
+        rho_prev += kprod<Cfg>(r0_hat[i], r0_hat[i]);
+        if constexpr (guarded) m0 = max_abs(max_abs(m0, tmp[i]), r0_hat[i]);
     }
+CUBIE_UNROLL
+    for (int i = 0; i < W; ++i) p[i] = r0_hat[i];
+    if constexpr (guarded) {
+        if (m0 > safe) {
+            rho_prev = L(0);
+CUBIE_UNROLL
+            for (int i = 0; i < W; ++i) {
+                const L ri = rhs[i] - clampc(tmp[i]);
+                r0_hat[i] = ri;
+                p[i] = clampc(ri);
+                rho_prev += clamp_pos(ri * ri);
+                m0 = max_abs(m0, ri);
+            }
+        }
+    }
+CUBIE_UNROLL
+    for (int i = 0; i < W; ++i) rhs[i] = r0_hat[i];
     L acc = P.krylov_norm2(rhs);
     bool converged = acc <= tol2;
     bool broken = false;
@@ -600,7 +657,7 @@ CUBIE_UNROLL
         // takes its square root in FP32
         real ndz;
         if constexpr (Cfg::newton_fast) ndz = real(dsqrt(float(norm2_dz)));
-        else ndz = real(dsqrt(norm2_dz));
+        else ndz = ssqrt<Cfg>(norm2_dz);
         const bool judged = lin == ST_SUCCESS;
         // FP32 Krylov solves of the mixed mode (single-stage Newton
         // families): a solve that ends in a BiCGSTAB breakdown (the
@@ -621,7 +678,7 @@ CUBIE_UNROLL
         const real ndz_prev_safe = history ? ndz_prev : real(1);
         real ratio;
         if constexpr (Cfg::newton_fast) ratio = real(float(ndz) * __builtin_amdgcn_rcpf(float(ndz_prev_safe)));
-        else ratio = ndz / ndz_prev_safe;
+        else ratio = sdiv<Cfg>(ndz, ndz_prev_safe);
         const real theta = history ? pmax(theta_decay * prev_theta, ratio) : prev_theta;
         const bool small_first = (iteration == 1) && (ndz < first_bound);
         const bool eta_accept = (theta < real(1)) && (theta * ndz < kappa * (real(1) - theta));
@@ -885,7 +942,7 @@ CUBIE_UNROLL
             // the tolerance (a weight, not a value the solution depends on)
             real r;
             if constexpr (Cfg::newton_fast) r = vals[i] * real(__builtin_amdgcn_rcpf(float(tol)));
-            else r = vals[i] / tol;
+            else r = sdiv<Cfg>(vals[i], tol);
             nrm2 += r * r;
         }
         return nrm2 * real(Cfg::inv_n);

@@ -117,7 +117,7 @@ CUBIE_UNROLL
                                         int* counters) {
         const real current_time = time;
         const real end_time = current_time + dt;
-        const real inv_dt = real(1) / dt;
+        const real inv_dt = sdiv<Cfg>(real(1), dt);
         const real* params = ctx.params.data();
 
         // Jacobian at the step start, in the linear-solve precision
@@ -161,7 +161,7 @@ CUBIE_UNROLL
 CUBIE_UNROLL
         for (int i = 0; i < n; ++i) {
             const L tol = L(Cfg::krylov_atol[i]) + L(Cfg::krylov_rtol[i]) * dabs(state_l[i]);
-            kw[i] = L(1) / pmax(tol, L(1e-16));
+            kw[i] = sdiv<Cfg>(L(1), pmax(tol, L(1e-16)));
         }
         Prob P;
         P.kw = kw.data();
