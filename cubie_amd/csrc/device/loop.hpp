@@ -455,8 +455,12 @@ __device__ __forceinline__ void integrate_persistent(const cubie_solve_args& a) 
     bool active = run < a.n_runs;
     if (active) it.begin(a, run);
     while (__any(active ? 1 : 0)) {
+        // step until a lane of the wavefront finishes: the queue and the
+        // start of a run stay out of the loop that does the work
         bool done = false;
-        if (active) done = it.advance(a);
+        do {
+            if (active) done = it.advance(a);
+        } while (!__any(done ? 1 : 0));
         if (active && done) it.finish(a);
         // Lanes that just finished take the next system of the batch.
         const long long next = grab_runs(a.work_counter, active && done);
