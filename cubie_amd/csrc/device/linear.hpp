@@ -122,12 +122,12 @@ __device__ __forceinline__ T ssqrt(T x) {
     return dsqrt(x);
 }
 
-// Krylov value clamps and divisions. The reference clamps every Krylov
-// vector and inner product to +-1e16 (FP32) / 1e150 (FP64) against overflow.
-// The compensated mode's FP32 solves (Cfg::krylov_fast) skip the clamps
-// (an overflowing solve returns a non-finite correction, which fails the
-// Newton pass; the step is then repeated with direct FP64 solves); in
-// production builds (Cfg::krylov_rcp) they also divide by the hardware
+// Krylov divisions. The reference clamps every Krylov vector and inner
+// product to +-1e16 (FP32) / 1e150 (FP64) against overflow (clampc, clamp_pos
+// in bicgstab_solve). The compensated mode's FP32 solves (Cfg::krylov_fast)
+// skip the clamps (an overflowing solve returns a non-finite correction, which
+// fails the Newton pass; the step is then repeated with direct FP64 solves);
+// in production builds (Cfg::krylov_rcp) they also divide by the hardware
 // reciprocal, parity builds keep IEEE division.
 template <typename Cfg, typename T>
 __device__ __forceinline__ T kdiv(T a, T b) {
