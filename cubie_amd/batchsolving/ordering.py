@@ -29,27 +29,37 @@ def morton_order(columns: List["object"]):
     """Permutation (int64 tensor on the columns' device) sorting the runs by
     the Morton key of the given (n_runs,) float tensors."""
     import torch
+    if not columns:
+        return torch.arange(0)
+    n = int(columns[0].numel())
+    dev = columns[0].device
+    wide = torch.stack([c.to(torch.float64).reshape(-1) for c in columns])
+    # every column's range in one transfer to the host
+    ranges = torch.stack((wide.amin(1), wide.amax(1))).tolist()
     cols = []
-    n = int(columns[0].numel()) if columns else 0
-    dev = columns[0].device if columns else None
-    if columns:
-        wide = [c.to(torch.float64) for c in columns]
-        # every column's range in one transfer to the host
-        ranges = torch.stack([torch.stack((c.min(), c.max(), c.abs().max())) for c in wide])
-        for c, (lo, hi, top) in zip(wide, ranges.tolist()):
-            span = hi - lo
-            scale = max(top, 1e-300)
-            if span > 1e-12 * scale:
-                cols.append(((c - lo) / span, span / scale))
+    for k, (lo, hi) in enumerate(zip(*ranges)):
+        span = hi - lo
+        scale = max(abs(lo), abs(hi), 1e-300)
+        if span > 1e-12 * scale:
+            cols.append((k, lo, span, span / scale))
     if not cols:
         return torch.arange(n, device=dev)
-    cols.sort(key=lambda cs: -cs[1])
-    cols = [c for c, _ in cols[:9]]
+    cols.sort(key=lambda c: -c[3])
+    cols = cols[:9]
     d = len(cols)
     bits = min(21, 63 // d)
+    if dev.type == "cuda":
+        from ..runtime import native
+        key = torch.empty(n, dtype=torch.int64, device=dev)
+        with torch.cuda.device(dev):
+            native.morton_keys(wide, key, [c[0] for c in cols], [c[1] for c in cols],
+                               [c[2] for c in cols], bits,
+                               torch.cuda.current_stream().cuda_stream)
+        return torch.argsort(key, stable=True)
     levels = (1 << bits) - 1
     key = torch.zeros(n, dtype=torch.int64, device=dev)
-    qs = [torch.clamp((c * levels).round().to(torch.int64), 0, levels) for c in cols]
+    qs = [torch.clamp(((wide[k] - lo) / span * levels).round().to(torch.int64), 0, levels)
+          for k, lo, span, _ in cols]
     for b in range(bits - 1, -1, -1):
         for q in qs:
             key = (key << 1) | ((q >> b) & 1)

@@ -190,6 +190,11 @@ def lib() -> ctypes.CDLL:
         L.cubie_hip_runs_to_rows.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_longlong,
                                              ctypes.c_longlong, ctypes.c_int, ctypes.c_void_p]
         L.cubie_hip_runs_to_rows.restype = ctypes.c_int
+        L.cubie_hip_morton_keys.argtypes = [
+            ctypes.c_void_p, ctypes.c_longlong, ctypes.c_int, ctypes.c_int,
+            ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_double),
+            ctypes.POINTER(ctypes.c_double), ctypes.c_void_p, ctypes.c_void_p]
+        L.cubie_hip_morton_keys.restype = ctypes.c_int
         if L.cubie_hip_abi_version() != ABI_VERSION:
             raise CubieNativeError("libcubie_hip.so ABI version mismatch; rebuild it")
         _lib = L
@@ -218,6 +223,22 @@ def runs_to_rows(src, dst, n_runs: int, inner: int, stream) -> None:
     check(lib().cubie_hip_runs_to_rows(ctypes.c_void_p(src.data_ptr()),
                                        ctypes.c_void_p(dst.data_ptr()), n_runs, inner, esize,
                                        ctypes.c_void_p(stream)), "cubie_hip_runs_to_rows")
+
+
+def morton_keys(columns, keys, index, lo, span, bits: int, stream) -> None:
+    """Enqueue the Morton keys (include/cubie_order.h) of the rows ``index``
+    of a float64 (columns, n_runs) device tensor into an int64 one."""
+    import torch
+    n_cols, n_runs = len(index), int(columns.shape[1])
+    if (columns.dtype != torch.float64 or keys.dtype != torch.int64 or keys.numel() != n_runs
+            or not columns.is_contiguous() or not keys.is_contiguous()
+            or columns.device != keys.device or max(index) >= columns.shape[0]):
+        raise CubieNativeError("morton_keys: a contiguous float64 (columns, n_runs) matrix and "
+                               "n_runs int64 keys on one device are needed")
+    check(lib().cubie_hip_morton_keys(
+        ctypes.c_void_p(columns.data_ptr()), n_runs, n_cols, bits, (ctypes.c_int * n_cols)(*index),
+        (ctypes.c_double * n_cols)(*lo), (ctypes.c_double * n_cols)(*span),
+        ctypes.c_void_p(keys.data_ptr()), ctypes.c_void_p(stream)), "cubie_hip_morton_keys")
 
 
 def compile_source(source: str, options, name: str = "cubie_kernel.hip") -> bytes:
