@@ -360,8 +360,15 @@ class BatchSolverKernel:
         that rows are staged, as they are where the vectors live in the
         private segment: a step there costs so much traffic that staging is
         lost in it (20 states x 50,000 runs: 57 ms, of which the transpose
-        0.16 ms), while lanes that wait for one another are not (60 ms)."""
+        0.16 ms), while lanes that wait for one another are not (60 ms).
+
+        Without a save grid there are two rows, the first and the final
+        state, which each lane writes in place: the ring's vote on every step
+        and its LDS earn nothing then (Van der Pol, 1,048,576 uneven runs,
+        final state: 352 ms through the ring, 298 ms in place)."""
         if (kernel_mode or self.kernel_mode) != "plain" or not self._rows_out_of_step(adjoint):
+            return 0
+        if self.timing.save_last:
             return 0
         if KernelSpec.placement_of(self.buffer_placement, self.system, self.algorithm,
                                    self.precision, self.output_config,
@@ -384,7 +391,9 @@ class BatchSolverKernel:
                        block_size: Optional[int] = None) -> bool:
         """Whether per-row outputs are staged run-major (see outputs.hpp
         row_index) and transposed after the launch: rows out of step that no
-        ring takes."""
+        ring takes, but for the plain kernel's two rows without a save grid."""
+        if (kernel_mode or self.kernel_mode) == "plain" and self.timing.save_last:
+            return False
         return (self._rows_out_of_step(adjoint)
                 and not self.row_ring(adjoint, kernel_mode, block_size))
 

@@ -82,3 +82,21 @@ def test_save_table_and_runs_that_end_early():
     assert ended.any() and not ended.all()
     assert np.all(out["state"][-1][:, ended] == 0.0)
     assert np.all(out["state"][-1][:, ~ended].sum(axis=0) > 0.5)
+
+
+@pytest.mark.parametrize("n", [1, 63, 65, 257])
+def test_final_state_alone_is_written_in_place(n):
+    """Two rows a run and no save grid: the plain kernel writes them directly,
+    the same as the persistent kernel's staged and transposed ones."""
+    inits, params = lorenz_batch(n, seed=8)
+
+    def make(mode):
+        return ca.Solver(lorenz(np.float64), algorithm="dormand-prince-54", atol=1e-8,
+                         rtol=1e-6, output_types=["state", "time"], deterministic_pow=True,
+                         kernel_mode=mode)
+    a, b = make("plain"), make("persistent")
+    assert a.kernel.row_ring() == 0 and not a.kernel.run_major_rows()
+    assert b.kernel.run_major_rows()
+    ra, rb = (s.solve(inits, params, duration=0.5) for s in (a, b))
+    assert ra.state.shape == rb.state.shape and ra.state.shape[0] == 2
+    assert np.array_equal(ra.state, rb.state) and np.all(ra.status_codes == 0)
